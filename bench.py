@@ -126,7 +126,7 @@ STEP_HEADERS = ("zfv_internal.hpp", "zfv_physics.hpp", "zfv_mm.hpp", "zfv_step_c
 KERNEL_FILES = {"tile": "zfv_tile.hip", "grad_pred": "zfv_kernels.hip", "corr": "zfv_kernels.hip",
                 "flux1": "zfv_kernels.hip", "k3_grad_pred": "zfv_3d.hip", "k3_corr": "zfv_3d.hip",
                 "k3_flux1": "zfv_3d.hip"}
-KERNEL_HEADERS = {"k3_grad_pred": ("zfv_3d.hpp",), "k3_corr": ("zfv_3d.hpp",), "k3_flux1": ("zfv_3d.hpp",)}
+KERNEL_HEADERS = {"tile": ("zfv_tile.hpp", "zfv_pair.hpp"), "k3_grad_pred": ("zfv_3d.hpp",), "k3_corr": ("zfv_3d.hpp",), "k3_flux1": ("zfv_3d.hpp",)}
 
 
 def kernel_sources_sha(kernel):

@@ -1,0 +1,94 @@
+"""The tiled kernels beyond the HLLC step that test_tile_gpu.py covers, against
+the one-thread-per-cell kernels on the same meshes, bit for bit (NaNs in the
+same places): the HLL and Rusanov MUSCL steps and the first-order steps, at the
+edges of a tile (62 cells by 2, 6, 10 or 14 rows) and on every kind of side;
+the shape that the library picks for a mesh's size; and states with NaN,
+infinite and vacuum cells.
+"""
+import numpy as np
+import pytest
+
+from test_tile_gpu import assert_same, quadrants
+
+pytestmark = pytest.mark.gpu
+
+GAMMA = 1.4
+SIDES = [(2, 2, 2, 2), (1, 1, 1, 1), (3, 3, 3, 3), (3, 2, 1, 3), (2, 3, 3, 1)]
+
+
+def pair(zfv, nx, ny, bounds, acc, flux, limiter="MC", shape=None):
+    out = []
+    for tiled in (False, True):
+        ctx = zfv.Context()
+        ctx.mesh_rectangle(nx, ny, bounds=bounds)
+        ctx.configure(acc=acc, flux=flux, limiter=limiter, cfl=0.5, gamma=GAMMA)
+        if not tiled:
+            for stage in range(3):
+                ctx.set_launch(stage, zfv.CELL, 256)
+        elif shape:
+            ctx.set_launch(1, zfv.TILE, shape)
+        ctx.set_state(*quadrants(nx, ny, 11))
+        out.append(ctx)
+    return out
+
+
+def equal(a, b, what):
+    for k, (x, y) in enumerate(zip(a, b)):
+        assert np.array_equal(x, y, equal_nan=True), f"{what}: component {k}"
+
+
+def steps_equal(ref, til, steps, what):
+    for k in range(steps):
+        ref.step(1)
+        til.step(1)
+        assert ref.dt() == til.dt(), f"{what}: dt of step {k}"
+        assert_same(ref.state(), til.state(), f"{what}: step {k}")
+        assert np.array_equal(ref.wait(), til.wait()), what
+
+
+@pytest.mark.parametrize("acc,flux", [(1, "hllc"), (1, "hll"), (1, "rusanov"), (2, "hll"), (2, "rusanov")])
+@pytest.mark.parametrize("bounds", SIDES)
+@pytest.mark.parametrize("nx,ny", [(1, 1), (2, 62), (3, 63), (7, 125), (33, 64)])
+def test_tiled_equals_cell_kernels(zfv, acc, flux, bounds, nx, ny):
+    ref, til = pair(zfv, nx, ny, bounds, acc, flux)
+    steps_equal(ref, til, 3, f"{acc} {flux} {bounds} {nx}x{ny}")
+
+
+@pytest.mark.parametrize("acc", [1, 2])
+@pytest.mark.parametrize("nx,ny", [(40, 40), (200, 200), (330, 280), (520, 390), (700, 900)])
+def test_every_default_shape(zfv, acc, nx, ny):
+    ref, til = pair(zfv, nx, ny, (2, 1, 3, 3), acc, "hllc")
+    steps_equal(ref, til, 2, f"{acc} {nx}x{ny}")
+
+
+@pytest.mark.parametrize("acc", [1, 2])
+@pytest.mark.parametrize("flux", ["hllc", "hll", "rusanov"])
+@pytest.mark.parametrize("limiter", ["MC", "minmod", "vanLeer"])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf, 0.0, 1e-310, 1e300])
+def test_cells_that_are_no_state(zfv, acc, flux, limiter, value):
+    """One field of a few cells out of any range (a NaN wave speed on one side
+    of a face, an empty cell, overflow in the gradient), inside, at a tile's
+    edge and at a wall.  Two steps: the second sees what the first left."""
+    nx, ny = 19, 70
+    for field in range(4):
+        ref, til = pair(zfv, nx, ny, (1, 2, 1, 2), acc, flux, limiter)
+        st = [a.copy() for a in quadrants(nx, ny, 5)]
+        for cell in (5 * ny + 20, 6 * ny + 61, 18 * ny + 69, 0):
+            st[field][cell] = value
+        for k in range(2):
+            got = []
+            for ctx in (ref, til):
+                if k == 0:
+                    ctx.set_state(*st)
+                ctx.step(1)
+                code = 0
+                try:
+                    ctx.synchronize()
+                except zfv.ZfvError as e:
+                    code = str(e)
+                out = [np.zeros(nx * ny) for _ in range(5)]
+                zfv.lib().zfv_state_download(ctx.h, *[zfv._ptr(a) for a in out])   # reports the sticky error too
+                got.append((code, out, ctx.wait()))
+            assert got[0][0] == got[1][0]
+            equal(got[0][1], got[1][1], f"field {field} step {k}")
+            assert np.array_equal(got[0][2], got[1][2])

@@ -21,6 +21,7 @@ SOURCES = [
     os.path.join(HERE, "csrc", "zfv_mm.hip"),
     os.path.join(HERE, "csrc", "zfv_order.hip"),
     os.path.join(HERE, "csrc", "zfv_tile.hip"),
+    os.path.join(HERE, "csrc", "zfv_tile_flux.hip"),
     os.path.join(HERE, "csrc", "zfv_transfer.hip"),
     os.path.join(HERE, "csrc", "zfv_3d.hip"),
     os.path.join(HERE, "csrc", "zfv_3d.cpp"),
@@ -33,6 +34,8 @@ HEADERS = [
     os.path.join(HERE, "csrc", "zfv_adjoint_ops.hpp"),
     os.path.join(HERE, "csrc", "zfv_step_common.hpp"),
     os.path.join(HERE, "csrc", "zfv_step_faces.hpp"),
+    os.path.join(HERE, "csrc", "zfv_pair.hpp"),
+    os.path.join(HERE, "csrc", "zfv_tile.hpp"),
     os.path.join(HERE, "csrc", "zfv_mm.hpp"),
     os.path.join(HERE, "csrc", "zfv_3d.hpp"),
     os.path.join(ROOT, "include", "zfv.h"),

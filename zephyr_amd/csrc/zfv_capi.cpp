@@ -148,15 +148,19 @@ struct zfv_ctx {
         bool ok = false;
         int n_probs = 0;
         int n_tiles[kTileVariants] = {0, 0, 0};
+        bool shared = false;      // every inner face has one geometry seen from both cells: the tiled kernels run
+        int n_rows = 0;
+        TileProb one{};           // the first problem
         DBuf<TileProb> prob;
         DBuf<TileCol> col;
-        DBuf<TileRow> row;
+        DBuf<double> row;         // [kTileRowAll][n_rows]
     } tiles;
     int tile_variant = 0;
     bool tile_persistent = false;   // tiled step by persistent workgroups (else one workgroup per tile)
     // The tiled step does not store its gradients: after one, the gradients
     // of the last step are recomputed on demand from its input (layer 1 - cur).
     bool grad_pending = false;
+    bool flux1_tile = true;     // first-order steps may run the tiled kernel (no layout was chosen for them)
 
     // batch of independent problems (nseg > 1): padded cell offsets, valid
     // cell counts, device tables of the kernels' Tile lookup
@@ -309,19 +313,22 @@ struct zfv_ctx {
         TileMesh T;
         T.n_probs = tiles.n_probs;
         for (int v = 0; v < kTileVariants; ++v) T.n_tiles[v] = tiles.n_tiles[v];
+        T.one = tiles.one;
         T.prob = tiles.prob.p;
         T.col = tiles.col.p;
         T.row = tiles.row.p;
+        T.row_stride = tiles.n_rows;
         T.vol = vol.p;
         T.h = h.p;
         return T;
     }
-    // Whether the steps run the tiled kernel: structured rectangles, MUSCL
-    // with HLLC, the state in the mesh's order.
-    bool tile_step() const {
-        return tiles.ok && prm.acc == 2 && prm.flux == ZFV_HLLC && layout[1] == kLayoutTile && !co.state &&
-               !prm.axial;
+    // Whether a tiled kernel covers the scheme: structured rectangles, HLLC,
+    // HLL or Rusanov, the state in the mesh's order.
+    bool tile_covers() const {
+        return tiles.ok && tiles.shared && tile_flux_built(prm.flux) && !co.state && !prm.axial;
     }
+    // ... and the MUSCL step runs it.
+    bool tile_step() const { return tile_covers() && prm.acc == 2 && layout[1] == kLayoutTile; }
     // Launch configuration of the gradient kernel when it runs on its own.
     int gp_layout() const { return layout[1] == kLayoutTile ? kLayoutCell : layout[1]; }
     int gp_block() const { return layout[1] == kLayoutTile ? kBlock : block[1]; }
@@ -392,9 +399,11 @@ bool build_tiles(zfv_ctx* ctx, const std::vector<int>& code, const std::vector<d
     const HostMesh& m = ctx->hm;
     const size_t n = (size_t)m.n;
     std::vector<TileProb> probs;
+    struct Side { double cx, cy, fx[4], fy[4], w[4], a[4]; };
     std::vector<TileCol> cols;
-    std::vector<TileRow> rows;
-    int tile0[kTileVariants] = {0, 0, 0};
+    std::vector<double> rows[kTileRowAll];
+    bool shared = true;
+    int tile0[kTileVariants] = {};
     for (const auto& R : ctx->rects) {
         const int nx = R.nx, ny = R.ny, off = R.off;
         if (nx < 1 || ny < 1 || (size_t)off + (size_t)nx * ny > n) return false;
@@ -408,7 +417,7 @@ bool build_tiles(zfv_ctx* ctx, const std::vector<int>& code, const std::vector<d
             tile0[v] += ((nx + kTileRows[v] - 1) / kTileRows[v]) * P.tiles_j;
         }
         P.col = (int)cols.size();
-        P.row = (int)rows.size();
+        P.row = (int)rows[0].size();
         const int c00 = off, cLast = off + (nx - 1) * ny + (ny - 1);
         P.t[0] = code[c00] & 7;
         P.t[1] = (code[cLast] >> 4) & 7;
@@ -418,19 +427,20 @@ bool build_tiles(zfv_ctx* ctx, const std::vector<int>& code, const std::vector<d
             if (P.t[s] != SC_PERIODIC && P.t[s] != SC_WALL && P.t[s] != SC_COPY) return false;
         P.per[0] = P.t[0] == SC_PERIODIC && P.t[1] == SC_PERIODIC;
         P.per[1] = P.t[2] == SC_PERIODIC && P.t[3] == SC_PERIODIC;
-        auto W = [&](int s, size_t c) { return w[(size_t)s * n + c]; };
-        for (int i = 0; i < nx; ++i) {
-            const size_t c = (size_t)off + (size_t)i * ny, f = 8 * c;
-            cols.push_back(TileCol{m.cx[c], m.fcx[f + 0], m.fcx[f + 1], m.fcx[f + 2], m.fcx[f + 3], W(0, c), W(1, c),
-                                   m.area[f + 2], m.area[f + 3]});
-        }
-        for (int j = 0; j < ny; ++j) {
-            const size_t c = (size_t)off + j, f = 8 * c;
-            rows.push_back(TileRow{m.cy[c], m.fcy[f + 0], m.fcy[f + 1], m.fcy[f + 2], m.fcy[f + 3], W(2, c), W(3, c),
-                                   m.area[f + 0], m.area[f + 1]});
-        }
-        const TileCol* C = &cols[P.col];
-        const TileRow* Rw = &rows[P.row];
+        // the first cell of each column / row
+        auto side = [&](size_t c) {
+            Side S{m.cx[c], m.cy[c], {}, {}, {}, {}};
+            for (int s = 0; s < 4; ++s) {
+                S.fx[s] = m.fcx[8 * c + s];
+                S.fy[s] = m.fcy[8 * c + s];
+                S.w[s] = w[(size_t)s * n + c];
+                S.a[s] = m.area[8 * c + s];
+            }
+            return S;
+        };
+        std::vector<Side> C(nx), Rw(ny);
+        for (int i = 0; i < nx; ++i) C[i] = side((size_t)off + (size_t)i * ny);
+        for (int j = 0; j < ny; ++j) Rw[j] = side((size_t)off + j);
         for (int i = 0; i < nx; ++i)
             for (int j = 0; j < ny; ++j) {
                 const size_t c = (size_t)off + (size_t)i * ny + j, f = 8 * c;
@@ -450,27 +460,74 @@ bool build_tiles(zfv_ctx* ctx, const std::vector<int>& code, const std::vector<d
                 for (int sl = 0; sl < 4; ++sl)
                     if (m.adj[f + sl] != adj[sl]) return false;
                 if (m.cx[c] != C[i].cx || m.cy[c] != Rw[j].cy) return false;
-                const double fx[4] = {C[i].fxL, C[i].fxR, C[i].fxB, C[i].fxT};
-                const double fy[4] = {Rw[j].fyL, Rw[j].fyR, Rw[j].fyB, Rw[j].fyT};
-                const double ar[4] = {Rw[j].aL, Rw[j].aR, C[i].aB, C[i].aT};
-                const double wt[4] = {C[i].wL, C[i].wR, Rw[j].wB, Rw[j].wT};
+                const double ar[4] = {Rw[j].a[0], Rw[j].a[1], C[i].a[2], C[i].a[3]};
+                const double wt[4] = {C[i].w[0], C[i].w[1], Rw[j].w[2], Rw[j].w[3]};
                 for (int sl = 0; sl < 4; ++sl) {
-                    if (m.fcx[f + sl] != fx[sl] || m.fcy[f + sl] != fy[sl] || m.area[f + sl] != ar[sl]) return false;
-                    if (W(sl, c) != wt[sl]) return false;
+                    if (m.fcx[f + sl] != C[i].fx[sl] || m.fcy[f + sl] != Rw[j].fy[sl] || m.area[f + sl] != ar[sl])
+                        return false;
+                    if (w[(size_t)sl * n + c] != wt[sl]) return false;
                 }
             }
+        // one axis of the LSM and the face offsets: lo / hi sides, centres c,
+        // face centres f, at position t of len (p + 2 (f - p) the mirror
+        // image of the cell beyond a side that is no inner one)
+        struct Axis { double dlo, dhi, A, olo, ohi, nlo, nhi; };
+        auto axis = [](int t, int len, double c, double clo, double chi, double flo, double fhi, double wlo, double whi,
+                       bool per_lo, bool per_hi) {
+            Axis X;
+            const double mlo = c + 2.0 * (flo - c), mhi = c + 2.0 * (fhi - c);
+            X.dlo = (t > 0 ? clo : mlo) - c;
+            X.dhi = (t < len - 1 ? chi : mhi) - c;
+            X.A = 0.0 + (wlo * X.dlo) * X.dlo;
+            X.A = X.A + (whi * X.dhi) * X.dhi;
+            X.olo = flo - c;
+            X.ohi = fhi - c;
+            X.nlo = t > 0 ? flo - clo : (per_lo ? flo - mlo : X.olo);
+            X.nhi = t < len - 1 ? fhi - chi : (per_hi ? fhi - mhi : X.ohi);
+            return X;
+        };
+        std::vector<Axis> ax(nx), ay(ny);
+        for (int i = 0; i < nx; ++i)
+            ax[i] = axis(i, nx, C[i].cx, i > 0 ? C[i - 1].cx : 0.0, i < nx - 1 ? C[i + 1].cx : 0.0, C[i].fx[0],
+                         C[i].fx[1], C[i].w[0], C[i].w[1], P.t[0] == SC_PERIODIC, P.t[1] == SC_PERIODIC);
+        for (int j = 0; j < ny; ++j)
+            ay[j] = axis(j, ny, Rw[j].cy, j > 0 ? Rw[j - 1].cy : 0.0, j < ny - 1 ? Rw[j + 1].cy : 0.0, Rw[j].fy[2],
+                         Rw[j].fy[3], Rw[j].w[2], Rw[j].w[3], P.t[2] == SC_PERIODIC, P.t[3] == SC_PERIODIC);
+        for (int i = 0; i < nx; ++i) {
+            const Axis& X = ax[i];
+            const double oxB = C[i].fx[2] - C[i].cx, oxT = C[i].fx[3] - C[i].cx;
+            shared = shared && oxB == oxT && (i == nx - 1 || (X.nhi == ax[i + 1].olo && X.ohi == ax[i + 1].nlo));
+            cols.push_back(TileCol{X.dlo, X.dhi, C[i].w[0], C[i].w[1], X.A, X.olo, X.ohi, oxB, X.nlo, X.nhi,
+                                   C[i].a[2], C[i].a[3]});
+        }
+        for (int j = 0; j < ny; ++j) {
+            const Axis& Y = ay[j];
+            const double oyL = Rw[j].fy[0] - Rw[j].cy, oyR = Rw[j].fy[1] - Rw[j].cy;
+            shared = shared && oyL == oyR && (j == ny - 1 || (Y.nhi == ay[j + 1].olo && Y.ohi == ay[j + 1].nlo));
+            const double v[kTileRowAll] = {Y.dlo, Y.dhi, Rw[j].w[2], Rw[j].w[3], std::fabs(Y.A) < 1e-8 ? 1.0 : Y.A,
+                                           oyL, Y.olo, Y.ohi, Rw[j].a[0], Rw[j].a[1], Y.nlo, Y.nhi};
+            for (int q = 0; q < kTileRowAll; ++q) rows[q].push_back(v[q]);
+        }
         probs.push_back(P);
     }
     hipStream_t s = ctx->stream;
+    const size_t nr = rows[0].size();
     if (T.prob.alloc(probs.size()) != hipSuccess || T.col.alloc(cols.size()) != hipSuccess ||
-        T.row.alloc(rows.size()) != hipSuccess)
+        T.row.alloc(kTileRowAll * nr) != hipSuccess)
         return false;
     if (hipMemcpyAsync(T.prob.p, probs.data(), probs.size() * sizeof(TileProb), hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(T.col.p, cols.data(), cols.size() * sizeof(TileCol), hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(T.row.p, rows.data(), rows.size() * sizeof(TileRow), hipMemcpyHostToDevice, s) != hipSuccess)
+        hipMemcpyAsync(T.col.p, cols.data(), cols.size() * sizeof(TileCol), hipMemcpyHostToDevice, s) != hipSuccess)
         return false;
+    for (int q = 0; q < kTileRowAll; ++q)
+        if (hipMemcpyAsync(T.row.p + q * nr, rows[q].data(), nr * sizeof(double), hipMemcpyHostToDevice, s) !=
+            hipSuccess)
+            return false;
+    if (hipStreamSynchronize(s) != hipSuccess) return false;   // the host tables end here
     T.n_probs = (int)probs.size();
+    T.n_rows = (int)nr;
+    T.one = probs[0];
     for (int v = 0; v < kTileVariants; ++v) T.n_tiles[v] = tile0[v];
+    T.shared = shared;
     T.ok = true;
     return true;
 }
@@ -1629,6 +1686,46 @@ int zfv_grad_download(zfv_ctx* ctx, double* dx, double* dy) {
     return ZFV_OK;
 }
 
+constexpr int kCus = 256;   // compute units of the MI355X
+
+// Tile shape of the steps: the caller's or the autotuner's, else the one
+// whose workgroups load the fullest CU least: k workgroups on a CU take about
+// a + b k us of a step.  Few rows per tile spread a small mesh over more CUs,
+// many rows compute fewer halo rows.  Measured (MUSCL, HLLC, MC; us): 2 rows
+// 9.5, 16, 20, 25 at k = 1 to 4, 6 rows 14, 25, 35, 46, 10 rows 19, 38, 14 rows
+// 23, 48; first order 2 rows 8.3, 13, 16, 19, 6 rows 12, 19, 22, 10 rows 14, 24,
+// 14 rows 16, 28.
+static int tile_shape(const zfv_ctx* ctx, double* cost = nullptr) {
+    const bool muscl = ctx->prm.acc == 2;
+    if (ctx->layout_set[1] && muscl) return ctx->tile_variant;
+    static const double a2[kTileVariants] = {5.5, 1.5, -3.0, 5.5}, b2[kTileVariants] = {10.0, 18.5, 26.0, 4.9};
+    static const double a1[kTileVariants] = {7.0, 5.5, 4.0, 6.0}, b1[kTileVariants] = {5.2, 9.2, 12.4, 3.4};
+    const double *a = muscl ? a2 : a1, *b = muscl ? b2 : b1;
+    int best = 0;
+    double least = 0.0;
+    for (int v = 0; v < kTileVariants; ++v) {
+        const double t = a[v] + b[v] * ((ctx->tiles.n_tiles[v] + kCus - 1) / kCus);
+        if (v == 0 || t < least) {
+            best = v;
+            least = t;
+        }
+    }
+    if (cost) *cost = least;
+    return best;
+}
+
+// Whether a first-order step runs the tiled kernel.  Rusanov and HLL always
+// (at 1361 x 1023 58 us against 79); HLLC, whose faces keep more registers,
+// up to the size from where the one-thread-per-cell kernel, about 13 us +
+// 53 us per million cells, is the faster one (1 M cells: 66 us against 76).
+static bool tile_first(const zfv_ctx* ctx) {
+    if (!ctx->tile_covers() || ctx->prm.acc != 1 || !ctx->flux1_tile) return false;
+    if (ctx->prm.flux != ZFV_HLLC) return true;
+    double cost = 0.0;
+    (void)tile_shape(ctx, &cost);
+    return cost < 13.0 + 53.0e-6 * ctx->hm.n;
+}
+
 // SmFluid::update x n_steps (sm_fluid.cpp:81-102).
 // One SmFluid::update (sm_fluid.cpp:81-102) enqueued on the context stream.
 static int step_once(zfv_ctx* ctx) {
@@ -1638,7 +1735,11 @@ static int step_once(zfv_ctx* ctx) {
     StepCtl ctl = make_ctl(ctx);
     const int nxt = (ctx->cur + 1) % 2;   // layers 0/1 alternate as init/next, 2 is half
     DevState in = ctx->layer(ctx->cur), out = ctx->layer(nxt);
-    if (P.acc == 1) {
+    if (tile_first(ctx)) {
+        ZFV_HIP(timed(ctx, "flux1", [&] {
+            return launch_tile_flux1(P.flux, tile_shape(ctx), ctx->tmesh(), in, out, eos, ctl, ctx->stream);
+        }));
+    } else if (P.acc == 1) {
         ZFV_HIP(timed(ctx, "flux1", [&] {
             return launch_flux1(P.flux, ctx->layout[0], ctx->block[0], M, in, out, eos, ctl, ctx->stream);
         }));
@@ -1647,8 +1748,8 @@ static int step_once(zfv_ctx* ctx) {
         int* w_out = ctx->wait[1 - ctx->wcur].p;
         const TileMesh T = ctx->tmesh();
         ZFV_HIP(timed(ctx, "tile", [&] {
-            return launch_tile_step(P.limiter, ctx->tile_variant, ctx->tile_persistent, T, in, out, w_in, w_out, eos,
-                                    ctl, ctx->stream);
+            return launch_tile_step(P.flux, P.limiter, tile_shape(ctx), ctx->tile_persistent, T, in, out, w_in, w_out,
+                                    eos, ctl, ctx->stream);
         }));
         ctx->wcur = 1 - ctx->wcur;
         ctx->grad_pending = true;   // the step's gradients were not stored
@@ -2994,7 +3095,7 @@ int zfv_limiter_from_name(const char* orig) {
 static bool valid_block(int b) { return b == 128 || b == 256 || b == 512; }
 
 static int tile_variant_of(int threads) {
-    for (int v = 0; v < kTileVariants; ++v)
+    for (int v = 0; v < kTileShapes; ++v)
         if (threads == (kTileRows[v] + 2) * 64) return v;
     return -1;
 }
@@ -3023,6 +3124,7 @@ int zfv_set_launch(zfv_ctx* ctx, int stage, int layout, int block) {
     ctx->layout[stage] = layout;
     if (block) ctx->block[stage] = block;
     ctx->layout_set[stage] = true;
+    if (stage == 0) ctx->flux1_tile = false;
     ctx->graphs_clear();
     return ZFV_OK;
 }
@@ -3121,16 +3223,24 @@ int zfv_autotune(zfv_ctx* ctx, int reps, double* ms_out) {
         ctx->layout[st] = bl;
         ctx->block[st] = blocks[bb];
         ctx->layout_set[st] = true;
+        if (st == 0 && ctx->tile_covers()) {   // the tiled first-order step against the best layout
+            const TileMesh T = ctx->tmesh();
+            const int v = tile_shape(ctx);
+            double ms = 0.0;
+            r = time_it([&] { return launch_tile_flux1(P.flux, v, T, in, out, eos, ctl, s); }, ms);
+            if (r) return r;
+            ctx->flux1_tile = ms < t[0][bl][bb];
+        }
     }
     // the tiled step (one kernel for the whole step) against the best pair
     // of gradient and corrector kernels
-    if (P.acc == 2 && P.flux == ZFV_HLLC && ctx->tiles.ok && !ctx->co.state) {
+    if (P.acc == 2 && ctx->tile_covers()) {
         // [1][tile][v]: one workgroup per tile; [2][tile][v]: persistent workgroups
         const TileMesh T = ctx->tmesh();
         int bv = 0, bp = 0;
-        for (int pers = 0; pers < 2; ++pers)
-            for (int v = 0; v < kTileVariants; ++v) {
-                r = time_it([&] { return launch_tile_step(P.limiter, v, pers != 0, T, in, out, w_in, w_out, eos, ctl, s); },
+        for (int pers = 0; pers < (P.flux == ZFV_HLLC ? 2 : 1); ++pers)
+            for (int v = 0; v < kTileShapes; ++v) {
+                r = time_it([&] { return launch_tile_step(P.flux, P.limiter, v, pers != 0, T, in, out, w_in, w_out, eos, ctl, s); },
                             t[1 + pers][kLayoutTile][v]);
                 if (r) return r;
                 if (t[1 + pers][kLayoutTile][v] < t[1 + bp][kLayoutTile][bv]) {

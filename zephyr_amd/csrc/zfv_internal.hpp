@@ -195,18 +195,29 @@ hipError_t launch_totals(const DevMesh& M, const DevState& z, double* partial, i
 // same values the slot arrays hold.  The tiled MUSCL step reads the state,
 // the isolation counters, volume and incircle per cell and the geometry from
 // the tables.
-struct TileCol {   // column i: centre x; face-centre x of slots L, R, B, T; weights of L, R; areas of B, T
-    double cx, fxL, fxR, fxB, fxT, wL, wR, aB, aT;
+// Differences that the step forms from centres and face centres are formed
+// here once, by the same subtractions.
+struct TileCol {   // column i
+    double drL, drR, wL, wR;    // LSM offsets along x of slots L, R, and their weights
+    double A00;                 // the LSM matrix's xx entry
+    double oxL, oxR, ox;        // face centre - cell centre, x component: slots L, R, and B / T
+    double nL, nR;              // ... of the cell across L / R at its mirror image (periodic sides)
+    double aB, aT;              // areas of slots B, T
 };
-struct TileRow {   // row j: centre y; face-centre y of slots L, R, B, T; weights of B, T; areas of L, R
-    double cy, fyL, fyR, fyB, fyT, wB, wT, aL, aR;
+// Row j, [kTileRowAll][row_stride]: the same along y (drB, drT, wB, wT, A11,
+// oy of slots L / R, oyB, oyT, areas of L, R; nB, nT).  The first kTileRowQ
+// are staged in LDS per tile.
+enum TileRowQuantity {
+    kRowDrB, kRowDrT, kRowWB, kRowWT, kRowA11, kRowOy, kRowOyB, kRowOyT, kRowAL, kRowAR, kTileRowQ,
+    kRowNB = kTileRowQ, kRowNT, kTileRowAll
 };
 // Tile shapes: kTileJ output cells along j (64-lane wavefronts with a halo
 // lane on each side) by kTileRows[v] along i, with (rows + 2) wavefronts
-// per workgroup (one per row of the tile and its two halo rows).
+// per workgroup (one per row of the tile and its two halo rows).  The first
+// kTileShapes can be chosen by the caller.
 constexpr int kTileJ = 62;
-constexpr int kTileVariants = 3;
-constexpr int kTileRows[kTileVariants] = {6, 10, 14};
+constexpr int kTileVariants = 4, kTileShapes = 3;
+constexpr int kTileRows[kTileVariants] = {6, 10, 14, 2};
 struct TileProb {
     int off, nx, ny;     // first cell, columns, rows
     int tiles_j;         // tiles along j
@@ -220,16 +231,23 @@ struct TileMesh {
     int n_tiles[kTileVariants];
     const TileProb* __restrict__ prob;
     const TileCol* __restrict__ col;
-    const TileRow* __restrict__ row;
+    const double* __restrict__ row;   // [kTileRowAll][row_stride]
+    int row_stride;
     const double* __restrict__ vol;
     const double* __restrict__ h;
+    TileProb one;   // the problem of a mesh that is not a batch: kernel arguments instead of a load of prob
 };
-// One MUSCL + HLLC step (gradient, limiting, predictor, corrector and the
-// next step's CFL candidate) per tile, intermediate values in LDS.
-// variant: the tile shape (kTileRows); workgroups of (kTileRows[v] + 2) * 64 threads.
-hipError_t launch_tile_step(int limiter, int variant, bool persistent, const TileMesh& T, const DevState& in,
-                            const DevState& out, const int* wait_in, int* wait_out, const Eos& eos,
-                            const StepCtl& ctl, hipStream_t s);
+// One MUSCL step (gradient, limiting, predictor, corrector and the next
+// step's CFL candidate) per tile, for the fluxes of tile_flux_built (HLLC,
+// HLL, Rusanov); variant: the tile shape (kTileRows), workgroups of
+// (kTileRows[v] + 2) * 64 threads; persistent applies to HLLC.
+bool tile_flux_built(int flux);
+hipError_t launch_tile_step(int flux, int limiter, int variant, bool persistent, const TileMesh& T,
+                            const DevState& in, const DevState& out, const int* wait_in, int* wait_out,
+                            const Eos& eos, const StepCtl& ctl, hipStream_t s);
+// One first-order step per tile.
+hipError_t launch_tile_flux1(int flux, int variant, const TileMesh& T, const DevState& in, const DevState& out,
+                             const Eos& eos, const StepCtl& ctl, hipStream_t s);
 // Scratch of the no-allocation entry points (zfv_kernels.hip): 4 result
 // doubles, then up to kScratchBlocks workgroups' 4 partial sums (4 MiB).
 constexpr int kScratchBlocks = 131072;
