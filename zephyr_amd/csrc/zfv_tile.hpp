@@ -92,6 +92,14 @@ __device__ __forceinline__ int problem_of(const TileMesh& T, int b) {
     return lo;
 }
 
+// By value: both sources end in scalar registers, where a selected reference
+// would have to be one kind of memory.
+__device__ __forceinline__ TileProb problem(const TileMesh& T, int pid) {
+    TileProb P = T.one;
+    if (T.n_probs != 1) P = T.prob[pid];
+    return P;
+}
+
 // The value of lane l + 1 / lane l - 1 (DPP wave_shl:1 / wave_shr:1; the end
 // lane gets 0).  Every lane of the wavefront must be active.
 __device__ __forceinline__ double from_next(double v) {
@@ -203,7 +211,7 @@ template <int V, int TI>
 __device__ __forceinline__ Place place_of(const TileMesh& T, int b) {
     Place p;
     p.pid = T.n_probs == 1 ? 0 : problem_of<V>(T, b);
-    const TileProb& P = T.n_probs == 1 ? T.one : T.prob[p.pid];
+    const TileProb P = problem(T, p.pid);
     const int t = b - P.tile0[V];
     const int ti = t / P.tiles_j, tj = t - ti * P.tiles_j;
     p.nx = P.nx;
@@ -255,7 +263,7 @@ __device__ __forceinline__ void tile_body(const TileMesh& T, const DevState& in,
                                           double* rt, int* ws, double* red) {
     constexpr int NW = TI + 2, XS = NW * 64, ZS = (TI + 4) * kBJ;
     const Place p = place_of<V, TI>(T, b);
-    const TileProb& P = T.n_probs == 1 ? T.one : T.prob[p.pid];
+    const TileProb P = problem(T, p.pid);
     const double dt = step_dt(ctl, p.pid);
     tile_prologue(ctl, p, dt);
 
@@ -501,7 +509,7 @@ __device__ __forceinline__ void tile_flux1_body(const TileMesh& T, const DevStat
                                                 const Eos& eos, const StepCtl& ctl, int b, double* ex, double* red) {
     constexpr int NW = TI + 2, XS = NW * 64;
     const Place p = place_of<V, TI>(T, b);
-    const TileProb& P = T.n_probs == 1 ? T.one : T.prob[p.pid];
+    const TileProb P = problem(T, p.pid);
     const double dt = step_dt(ctl, p.pid);
     tile_prologue(ctl, p, dt);
     const int c = p.off + p.gi * p.ny + p.gj;
