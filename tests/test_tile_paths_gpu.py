@@ -2,8 +2,8 @@
 the one-thread-per-cell kernels on the same meshes, bit for bit (NaNs in the
 same places): the HLL and Rusanov MUSCL steps and the first-order steps, at the
 edges of a tile (62 cells by 2, 6, 10 or 14 rows) and on every kind of side;
-the shape that the library picks for a mesh's size; and states with NaN,
-infinite and vacuum cells.
+the shape that the library picks for a mesh's size; states with NaN, infinite
+and vacuum cells; and what a state upload leaves of the last step's gradients.
 """
 import numpy as np
 import pytest
@@ -92,3 +92,79 @@ def test_cells_that_are_no_state(zfv, acc, flux, limiter, value):
             assert got[0][0] == got[1][0]
             equal(got[0][1], got[1][1], f"field {field} step {k}")
             assert np.array_equal(got[0][2], got[1][2])
+
+
+def test_upload_keeps_the_last_steps_gradients(zfv):
+    """grad() after an upload is that of the last step, with the limiter the
+    step had, whatever is configured or stepped in between."""
+    for after in ("nothing", "limiter", "first order"):
+        ref, til = pair(zfv, 30, 70, (2, 2, 2, 2), 2, "hllc")
+        for ctx in (ref, til):
+            ctx.step(3)
+            ctx.set_state(*quadrants(30, 70, 12))
+            if after == "limiter":
+                ctx.configure(acc=2, flux="hllc", limiter="minmod", cfl=0.5, gamma=GAMMA)
+            elif after == "first order":
+                ctx.configure(acc=1, flux="hllc", limiter="MC", cfl=0.5, gamma=GAMMA)
+                ctx.step(2)
+        assert_same(ref.grad(), til.grad(), after)
+
+
+def test_gradients_after_graph_replays_and_batch_uploads(zfv):
+    sizes = [(20, 33), (7, 62), (3, 3)]
+    out = []
+    for tiled in (False, True):
+        ctx = zfv.Context()
+        ctx.batch_rectangles(sizes)
+        ctx.configure(acc=2, flux="hllc", limiter="MC", cfl=0.5, gamma=GAMMA)
+        if not tiled:
+            ctx.set_launch(1, zfv.CELL, 256)
+        ctx.graph_enable(True)
+        begin, count = ctx.batch_layout()
+        got = []
+        for seed in (1, 2, 3):
+            full = [np.full(ctx.n, 3.0 + k) for k in range(5)]
+            for p, (nx, ny) in enumerate(sizes):
+                for k, a in enumerate(quadrants(nx, ny, seed + p)):
+                    full[k][begin[p]:begin[p] + count[p]] = a
+            ctx.set_state(*full)
+            for n in (7, 6):
+                ctx.step(n)
+                got.append(ctx.state() + list(ctx.grad()))
+        out.append(got)
+    for a, b in zip(*out):
+        assert_same(a[:5], b[:5], "states, padding cells among them")
+        used = np.concatenate([np.arange(p, p + c) for p, c in zip(begin, count)])
+        assert_same([g[:, used] for g in a[5:]], [g[:, used] for g in b[5:]], "gradients")
+
+
+def test_device_copies_of_any_alignment(zfv):
+    """State up and down through device pointers, odd sizes and rows that do
+    not start on 16 bytes."""
+    import ctypes as C
+    hip = zfv.lib()   # the HIP runtime that the library itself is linked to
+    for nx, ny, shift in ((9, 7, 0), (8, 8, 0), (8, 8, 1), (64, 33, 1)):
+        n = nx * ny
+        ctx = zfv.Context()
+        ctx.mesh_rectangle(nx, ny)
+        ctx.configure(acc=2, flux="hllc", limiter="MC", cfl=0.5, gamma=GAMMA)
+        st = np.stack(quadrants(nx, ny, 3))
+        host = np.zeros((5, n + 3))
+        host[:, shift:shift + n] = st
+        bufs = [C.c_void_p() for _ in range(2)]
+        for b, h in zip(bufs, (host, np.zeros_like(host))):
+            assert hip.hipMalloc(C.byref(b), C.c_size_t(host.nbytes)) == 0
+            assert hip.hipMemcpy(b, C.c_void_p(h.ctypes.data), C.c_size_t(h.nbytes), 1) == 0
+        at = lambda b: [b.value + 8 * ((n + 3) * k + shift) for k in range(5)]   # noqa: E731
+        for _ in range(2):
+            ctx.set_state_device(at(bufs[0]))
+            assert zfv.lib().zfv_state_download_device(ctx.h, *[C.c_void_p(p) for p in at(bufs[1])]) == 0
+            back = np.ones_like(host)
+            assert hip.hipMemcpy(C.c_void_p(back.ctypes.data), bufs[1], C.c_size_t(back.nbytes), 2) == 0
+            assert np.array_equal(back, host)
+            dt = ctx.compute_dt()
+            ctx.step(2)
+            assert ctx.dt() > 0.0 and dt > 0.0
+        ctx.close()
+        for b in bufs:
+            assert hip.hipFree(b) == 0

@@ -160,6 +160,16 @@ struct zfv_ctx {
     // The tiled step does not store its gradients: after one, the gradients
     // of the last step are recomputed on demand from its input (layer 1 - cur).
     bool grad_pending = false;
+    // ... with the limiter that was set when a state upload followed the step
+    // (-1: none did, the limiter set when they are asked for)
+    int grad_limiter = -1;
+    // dt and error word of a synchronising call, in pinned host memory
+    struct Report {
+        double dt;
+        int err;
+    };
+    Report* report = nullptr;
+    bool slots_reset = false;   // the CFL slots hold +inf (state upload)
     bool flux1_tile = true;     // first-order steps may run the tiled kernel (no layout was chosen for them)
 
     // batch of independent problems (nseg > 1): padded cell offsets, valid
@@ -666,6 +676,7 @@ int upload_mesh(zfv_ctx* ctx) {
     ZFV_HIP(hipStreamSynchronize(s));
     ctx->graphs_clear();
     ctx->grad_pending = false;
+    ctx->slots_reset = false;
     if (!ctx->layout_set[1]) {   // default: the tiled step where it applies
         ctx->layout[1] = ctx->tiles.ok ? kLayoutTile : kLayoutCell;
         ctx->block[1] = ctx->tiles.ok ? (kTileRows[0] + 2) * 64 : kBlock;
@@ -703,16 +714,19 @@ int upload_mesh(zfv_ctx* ctx) {
 // solve), bit 1 inconsistent mesh after an adaptation; bits 2 and 3 are
 // notices for the adjoint (a cell in the robust isolation mode, a cell
 // isolated by the corrector), not errors of the step.
-int read_err(zfv_ctx* ctx) {
-    int e = 0;
-    ZFV_HIP(hipMemcpyAsync(&e, ctx->err.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    ZFV_HIP(hipStreamSynchronize(ctx->stream));
+int check_err(zfv_ctx* ctx, int e) {
     if (e & 2) {
         ctx->have_state = false;
         return fail(ZFV_ERR_STATE, "AMR apply produced an inconsistent mesh; state invalidated");
     }
     if (e & 1) return fail(ZFV_ERR_NUMERIC, "numeric error: a flux or Riemann solve produced NaN / did not converge");
     return ZFV_OK;
+}
+
+int read_err(zfv_ctx* ctx) {
+    ZFV_HIP(launch_report(nullptr, ctx->err.p, nullptr, &ctx->report->err, ctx->stream));
+    ZFV_HIP(hipStreamSynchronize(ctx->stream));
+    return check_err(ctx, ctx->report->err);
 }
 
 // Growth of the [rows][cap] device arrays to a larger capacity, keeping the
@@ -900,7 +914,9 @@ hipError_t timed(zfv_ctx* ctx, const char* name, F&& launch) {
 int ensure_dt(zfv_ctx* ctx) {
     if (ctx->dt_valid) return ZFV_OK;
     int rd = (int)(ctx->step_no % 3);
-    ZFV_HIP(launch_fill_u64(ctx->dtmin.p, 3 * ctx->nseg, 0x7ff0000000000000ULL, ctx->stream));
+    if (!ctx->slots_reset)
+        ZFV_HIP(launch_fill_u64(ctx->dtmin.p, 3 * ctx->nseg, 0x7ff0000000000000ULL, ctx->stream));
+    ctx->slots_reset = false;
     DevMesh M = ctx->smesh();
     DevState z = ctx->layer(ctx->cur);
     Eos eos = ctx->eos();
@@ -1108,7 +1124,10 @@ int zfv_create(int device, zfv_ctx** out) {
     }
     ctx->stream = ctx->own_stream;
     ctx->prm.max_dt = std::numeric_limits<double>::max();
-    if (ctx->dmax_dt.alloc(1) != hipSuccess || put_max_dt(ctx) != ZFV_OK) {
+    if (ctx->dmax_dt.alloc(1) != hipSuccess ||
+        hipHostMalloc((void**)&ctx->report, sizeof(zfv_ctx::Report), hipHostMallocDefault) != hipSuccess ||
+        put_max_dt(ctx) != ZFV_OK) {
+        if (ctx->report) (void)hipHostFree(ctx->report);
         (void)hipStreamDestroy(ctx->own_stream);
         delete ctx;
         return fail(ZFV_ERR_HIP, "context allocation failed");
@@ -1131,6 +1150,7 @@ int zfv_destroy(zfv_ctx* ctx) {
         (void)hipStreamDestroy(ctx->mm.side);
     }
     if (ctx->marks_total) (void)hipHostFree(ctx->marks_total);
+    if (ctx->report) (void)hipHostFree(ctx->report);
     hipStream_t s = ctx->own_stream;
     delete ctx;
     if (s) (void)hipStreamDestroy(s);
@@ -1431,9 +1451,10 @@ int zfv_batch_dt(zfv_ctx* ctx, double* dt) {
     int r = need_ready(ctx, false);
     if (r) return r;
     if (!dt) return fail(ZFV_ERR_ARG, "null output");
+    ZFV_HIP(launch_report(nullptr, ctx->err.p, nullptr, &ctx->report->err, ctx->stream));
     ZFV_HIP(hipMemcpyAsync(dt, ctx->dt_out.p, ctx->nseg * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     ZFV_HIP(hipStreamSynchronize(ctx->stream));
-    return read_err(ctx);
+    return check_err(ctx, ctx->report->err);
 }
 
 int zfv_mesh_n_cells(zfv_ctx* ctx, int32_t* n) {
@@ -1575,78 +1596,97 @@ int zfv_smf_set_max_dt(zfv_ctx* ctx, double max_dt) {
 
 static int materialize_grads(zfv_ctx* ctx);
 
-static int state_copy(zfv_ctx* ctx, const double* const* src, bool to_device, hipMemcpyKind kind) {
+// Whether the five rows lie in this device's own memory, where one kernel can
+// copy them (other memory goes through hipMemcpy, as before).
+static bool on_device(const zfv_ctx* ctx, const double* const* rows) {
+    for (int k = 0; k < 5; ++k) {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, rows[k]) != hipSuccess) {
+            (void)hipGetLastError();   // not a HIP allocation
+            return false;
+        }
+        if (a.type != hipMemoryTypeDevice || a.device != ctx->device) return false;
+    }
+    return true;
+}
+
+static int state_upload(zfv_ctx* ctx, const double* const* src, hipMemcpyKind kind) {
+    int r = need_ready(ctx, false);
+    if (r) return r;
+    r = to_mesh_order(ctx);
+    if (r) return r;
     const int n = ctx->hm.n;
     for (int k = 0; k < 5; ++k)
         if (!src[k]) return fail(ZFV_ERR_ARG, "null state array");
-    if (to_device) {   // the last step's input may be overwritten: its gradients first
-        int r = materialize_grads(ctx);
-        if (r) return r;
-    }
+    // The last tiled step's gradients are recomputed on demand from its input,
+    // layer 1 - cur, whose cells an upload leaves as they are.
+    if (ctx->grad_pending && ctx->grad_limiter < 0) ctx->grad_limiter = ctx->prm.limiter;
+    double *dst[5], *dst2[5];
     for (int k = 0; k < 5; ++k) {
-        double* d = ctx->st[ctx->cur][k].p;
-        if (to_device) ZFV_HIP(hipMemcpyAsync(d, src[k], n * sizeof(double), kind, ctx->stream));
-        else ZFV_HIP(hipMemcpyAsync(const_cast<double*>(src[k]), d, n * sizeof(double), kind, ctx->stream));
+        dst[k] = ctx->st[ctx->cur][k].p;
+        dst2[k] = ctx->st[1 - ctx->cur][k].p;
     }
     // A batch's padding cells are never written by the step kernels: give
-    // both alternating layers the uploaded values, so a download returns
-    // them whatever the parity of the step count.
-    if (to_device && ctx->nseg > 1)
+    // both alternating layers the uploaded values there, so a download
+    // returns them whatever the parity of the step count.
+    const DevMesh M = ctx->dmesh();
+    if (kind == hipMemcpyDeviceToDevice && on_device(ctx, src)) {
+        ZFV_HIP(launch_state_copy(src, dst, M.chunk_pid ? dst2 : nullptr, M, ctx->dtmin.p, 3 * ctx->nseg, nullptr,
+                                  nullptr, ctx->stream));
+        ctx->slots_reset = true;
+    } else {
         for (int k = 0; k < 5; ++k)
-            ZFV_HIP(hipMemcpyAsync(ctx->st[1 - ctx->cur][k].p, ctx->st[ctx->cur][k].p, n * sizeof(double),
-                                   hipMemcpyDeviceToDevice, ctx->stream));
+            ZFV_HIP(hipMemcpyAsync(dst[k], src[k], n * sizeof(double), kind, ctx->stream));
+        if (M.chunk_pid) ZFV_HIP(launch_state_copy(dst, nullptr, dst2, M, nullptr, 0, nullptr, nullptr, ctx->stream));
+        ctx->slots_reset = false;
+    }
     ZFV_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->have_state = true;
+    ctx->dt_valid = false;
     return ZFV_OK;
+}
+
+static int state_download(zfv_ctx* ctx, double* const* dst, hipMemcpyKind kind) {
+    int r = need_ready(ctx);
+    if (r) return r;
+    r = to_mesh_order(ctx);
+    if (r) return r;
+    const int n = ctx->hm.n;
+    for (int k = 0; k < 5; ++k)
+        if (!dst[k]) return fail(ZFV_ERR_ARG, "null state array");
+    double* src[5];
+    for (int k = 0; k < 5; ++k) src[k] = ctx->st[ctx->cur][k].p;
+    if (kind == hipMemcpyDeviceToDevice && on_device(ctx, dst)) {
+        ZFV_HIP(launch_state_copy(src, dst, nullptr, ctx->dmesh(), nullptr, 0, ctx->err.p, &ctx->report->err, ctx->stream));
+    } else {
+        for (int k = 0; k < 5; ++k)
+            ZFV_HIP(hipMemcpyAsync(dst[k], src[k], n * sizeof(double), kind, ctx->stream));
+        ZFV_HIP(launch_report(nullptr, ctx->err.p, nullptr, &ctx->report->err, ctx->stream));
+    }
+    ZFV_HIP(hipStreamSynchronize(ctx->stream));
+    return check_err(ctx, ctx->report->err);
 }
 
 int zfv_state_upload(zfv_ctx* ctx, const double* rho, const double* u, const double* v, const double* p,
                      const double* e) {
-    int r = need_ready(ctx, false);
-    if (r) return r;
-    r = to_mesh_order(ctx);
-    if (r) return r;
     const double* a[5] = {rho, u, v, p, e};
-    r = state_copy(ctx, a, true, hipMemcpyHostToDevice);
-    if (r) return r;
-    ctx->have_state = true;
-    ctx->dt_valid = false;
-    return ZFV_OK;
+    return state_upload(ctx, a, hipMemcpyHostToDevice);
 }
 
 int zfv_state_upload_device(zfv_ctx* ctx, const double* rho, const double* u, const double* v,
                             const double* p, const double* e) {
-    int r = need_ready(ctx, false);
-    if (r) return r;
-    r = to_mesh_order(ctx);
-    if (r) return r;
     const double* a[5] = {rho, u, v, p, e};
-    r = state_copy(ctx, a, true, hipMemcpyDeviceToDevice);
-    if (r) return r;
-    ctx->have_state = true;
-    ctx->dt_valid = false;
-    return ZFV_OK;
+    return state_upload(ctx, a, hipMemcpyDeviceToDevice);
 }
 
 int zfv_state_download(zfv_ctx* ctx, double* rho, double* u, double* v, double* p, double* e) {
-    int r = need_ready(ctx);
-    if (r) return r;
-    r = to_mesh_order(ctx);
-    if (r) return r;
-    const double* a[5] = {rho, u, v, p, e};
-    r = state_copy(ctx, a, false, hipMemcpyDeviceToHost);
-    if (r) return r;
-    return read_err(ctx);
+    double* a[5] = {rho, u, v, p, e};
+    return state_download(ctx, a, hipMemcpyDeviceToHost);
 }
 
 int zfv_state_download_device(zfv_ctx* ctx, double* rho, double* u, double* v, double* p, double* e) {
-    int r = need_ready(ctx);
-    if (r) return r;
-    r = to_mesh_order(ctx);
-    if (r) return r;
-    const double* a[5] = {rho, u, v, p, e};
-    r = state_copy(ctx, a, false, hipMemcpyDeviceToDevice);
-    if (r) return r;
-    return read_err(ctx);
+    double* a[5] = {rho, u, v, p, e};
+    return state_download(ctx, a, hipMemcpyDeviceToDevice);
 }
 
 int zfv_wait_upload(zfv_ctx* ctx, const int32_t* wait) {
@@ -1753,6 +1793,7 @@ static int step_once(zfv_ctx* ctx) {
         }));
         ctx->wcur = 1 - ctx->wcur;
         ctx->grad_pending = true;   // the step's gradients were not stored
+        ctx->grad_limiter = -1;
         ctx->co.grad = false;
     } else {
         DevGrad G{ctx->gdx.p, ctx->gdy.p};
@@ -1783,8 +1824,8 @@ static int materialize_grads(zfv_ctx* ctx) {
     if (!ctx->grad_pending) return ZFV_OK;
     const DevGrad G{ctx->gdx.p, ctx->gdy.p};
     const int prev = 1 - ctx->cur;
-    ZFV_HIP(launch_grad_pred(ctx->prm.limiter, false, ctx->gp_layout(), ctx->gp_block(), ctx->dmesh(),
-                             ctx->layer(prev), G, ctx->layer(2), ctx->wait[ctx->wcur].p, ctx->eos(), make_ctl(ctx),
+    const int limiter = ctx->grad_limiter < 0 ? ctx->prm.limiter : ctx->grad_limiter;
+    ZFV_HIP(launch_grad_pred(limiter, false, ctx->gp_layout(), ctx->gp_block(), ctx->dmesh(), ctx->layer(prev), G, ctx->layer(2), ctx->wait[ctx->wcur].p, ctx->eos(), make_ctl(ctx),
                              ctx->stream));
     ctx->grad_pending = false;
     ctx->co.grad = false;
@@ -1853,6 +1894,10 @@ int zfv_smf_step(zfv_ctx* ctx, int n_steps) {
     if (n_steps < 0) return fail(ZFV_ERR_ARG, "negative step count");
     r = to_curve_order(ctx);
     if (r) return r;
+    if (ctx->prm.acc == 1 && ctx->grad_limiter >= 0 && n_steps > 0) {
+        r = materialize_grads(ctx);   // a first-order step overwrites their input and brings none
+        if (r) return r;
+    }
     r = ensure_dt(ctx);
     if (r) return r;
     int it = 0;
@@ -1863,6 +1908,10 @@ int zfv_smf_step(zfv_ctx* ctx, int n_steps) {
             if (r) return r;
             ZFV_HIP(hipGraphLaunch(exec, ctx->stream));
             ctx->step_no += kGraphSteps;   // cur and wcur return to their values after 6 swaps
+            if (ctx->tile_step()) {        // as step_once leaves them (a replay does not run it)
+                ctx->grad_pending = true;
+                ctx->grad_limiter = -1;
+            }
             it += kGraphSteps;
         }
     }
@@ -1925,9 +1974,10 @@ int zfv_smf_dt(zfv_ctx* ctx, double* dt) {
     int r = need_ready(ctx, false);
     if (r) return r;
     if (!dt) return fail(ZFV_ERR_ARG, "null output");
-    ZFV_HIP(hipMemcpyAsync(dt, ctx->dt_out.p, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    ZFV_HIP(launch_report(ctx->dt_out.p, ctx->err.p, &ctx->report->dt, &ctx->report->err, ctx->stream));
     ZFV_HIP(hipStreamSynchronize(ctx->stream));
-    return read_err(ctx);
+    *dt = ctx->report->dt;
+    return check_err(ctx, ctx->report->err);
 }
 
 int zfv_smf_compute_grad(zfv_ctx* ctx) {
@@ -2119,6 +2169,7 @@ static int refine_impl(zfv_ctx* ctx, int max_level, int mode) {
     const bool carry_ok = !mm && co.mode == 1 && co.keys_ok && co.refined && co.epoch == ctx->mesh_epoch &&
                           co.cap == ctx->cap;
     co.perm_epoch = -1;
+    ctx->slots_reset = false;   // the derive pass fills the next step's slot
     ZFV_HIP(amr_mark(ctx->amesh(), ctx->s_marks.p, carry_ok ? co.perm.p : nullptr, s));
     r = scan3(ctx, ctx->s_marks.p, ctx->s_rank.p, n);
     if (r) return r;

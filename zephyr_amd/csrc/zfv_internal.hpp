@@ -168,6 +168,12 @@ hipError_t gather_rows(const double* src, double* dst, const int* idx, int n, in
 
 // Launchers (zfv_kernels.hip).
 hipError_t launch_fill_u64(unsigned long long* p, int count, unsigned long long v, hipStream_t s);
+// The mesh's cells of five state rows from src to dst (dst null:
+// not copied), and a batch's padding cells from src to dst2 (or null); the CFL
+// slots reset and the error word reported (pinned host memory) where given.
+hipError_t launch_state_copy(const double* const* src, double* const* dst, double* const* dst2, const DevMesh& M,
+                             unsigned long long* slots, int nslots, const int* err, int* report, hipStream_t s);
+hipError_t launch_report(const double* dt, const int* err, double* dt_out, int* err_out, hipStream_t s);
 hipError_t launch_dt(const DevMesh& M, const DevState& z, const Eos& eos, unsigned long long* slot, hipStream_t s);
 
 // Step-kernel layouts: one thread per cell, a lane quad per cell, or one
@@ -228,6 +234,7 @@ struct TileProb {
 };
 struct TileMesh {
     int n_probs;
+    TileProb one;   // the problem of a mesh that is not a batch: kernel arguments instead of a load of prob
     int n_tiles[kTileVariants];
     const TileProb* __restrict__ prob;
     const TileCol* __restrict__ col;
@@ -235,7 +242,6 @@ struct TileMesh {
     int row_stride;
     const double* __restrict__ vol;
     const double* __restrict__ h;
-    TileProb one;   // the problem of a mesh that is not a batch: kernel arguments instead of a load of prob
 };
 // One MUSCL step (gradient, limiting, predictor, corrector and the next
 // step's CFL candidate) per tile, for the fluxes of tile_flux_built (HLLC,

@@ -14,6 +14,8 @@
 // cells with cross-lane shuffles and LDS, then one 64-bit atomicMin on the bit
 // pattern (positive doubles order like unsigned integers).  NaN candidates
 // are dropped, as `temp < res` drops them in threads::min (utils/threads.h:292-352).
+#include <algorithm>
+
 #include "zfv_internal.hpp"
 #include "zfv_step_common.hpp"
 #include "zfv_step_faces.hpp"
@@ -75,12 +77,76 @@ __global__ void __launch_bounds__(256) k_fill_u64(unsigned long long* p, int cou
     if (i < count) p[i] = v;
 }
 
+// In a batch a workgroup takes its 256 cells (one problem); otherwise the
+// workgroups stride over the mesh, so that a large mesh ends in kDtBlocks
+// atomics on its one slot instead of one per 256 cells: these take about 12 ns
+// each, one after the other (66 us of a 1361 x 1023 mesh's reduction, whose
+// reads take 14).
+constexpr int kDtBlocks = 512;
 __global__ void __launch_bounds__(kMaxBlock) k_dt(DevMesh M, DevState z, Eos eos, unsigned long long* slot) {
     const Tile t = tile_of(M, (int)blockDim.x);
-    const int c = t.c0 + (int)threadIdx.x;
+    const int step = M.chunk_pid ? t.end : (int)(gridDim.x * blockDim.x);
     double cand = INFINITY;
-    if (c < t.end) cand = cell_dt(load_z(z, c), M.h[c], eos);
+    for (int c = t.c0 + (int)threadIdx.x; c < t.end; c += step) {
+        const double v = cell_dt(load_z(z, c), M.h[c], eos);
+        cand = (v < cand) ? v : cand;   // NaN never wins
+    }
     block_min_atomic(slot + 3 * t.pid, cand);
+}
+
+// The five rows of a state in one launch (at 64 x 48 cells five copies take
+// 13 us of GPU time, this 2): into dst, and a batch's padding cells into dst2,
+// each where given.  Also, where given: the CFL slots reset (nslots of them),
+// and the error word reported to pinned host memory.
+struct StateCopy {
+    const double* src[5];
+    double* dst[5];
+    double* dst2[5];
+    const int* chunk_pid;
+    const int* seg_end;
+    unsigned long long* slots;
+    int nslots;
+    const int* err;
+    int* report;
+};
+
+// PAIRS: n is even, every row lies on a 16-byte boundary, and there is no dst2.
+template <bool PAIRS>
+__global__ void __launch_bounds__(256) k_state_copy(StateCopy a, int n) {
+    const int first = (int)(blockIdx.x * blockDim.x + threadIdx.x), step = (int)(gridDim.x * blockDim.x);
+    if (PAIRS) {
+        for (int i = first; i < n >> 1; i += step) {
+            double2 v[5];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) v[k] = reinterpret_cast<const double2*>(a.src[k])[i];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) reinterpret_cast<double2*>(a.dst[k])[i] = v[k];
+        }
+    } else {
+        for (int i = first; i < n; i += step) {
+            double v[5];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) v[k] = a.src[k][i];
+            if (a.dst[0]) {
+#pragma unroll
+                for (int k = 0; k < 5; ++k) a.dst[k][i] = v[k];
+            }
+            if (a.dst2[0] && i >= a.seg_end[a.chunk_pid[i >> kChunkShift]]) {
+#pragma unroll
+                for (int k = 0; k < 5; ++k) a.dst2[k][i] = v[k];
+            }
+        }
+    }
+    for (int i = first; i < a.nslots; i += step) a.slots[i] = kInfBits;
+    if (a.report && first == 0) *a.report = *a.err;
+}
+
+// dt of the last step and the error word into pinned host memory.
+__global__ void __launch_bounds__(64) k_report(const double* dt, const int* err, double* dt_out, int* err_out) {
+    if (threadIdx.x == 0) {
+        if (dt) *dt_out = *dt;
+        *err_out = *err;
+    }
 }
 
 // SmFluid::fluxes, first order (sm_fluid.cpp:127-174), plus the next step's
@@ -1083,7 +1149,38 @@ hipError_t launch_fill_u64(unsigned long long* p, int count, unsigned long long 
 }
 
 hipError_t launch_dt(const DevMesh& M, const DevState& z, const Eos& eos, unsigned long long* slot, hipStream_t s) {
-    hipLaunchKernelGGL(k_dt, dim3(grid_cells(M.n, kBlock)), dim3(kBlock), 0, s, M, z, eos, slot);
+    int g = grid_cells(M.n, kBlock);
+    if (!M.chunk_pid && g > kDtBlocks) g = kDtBlocks;
+    hipLaunchKernelGGL(k_dt, dim3(g), dim3(kBlock), 0, s, M, z, eos, slot);
+    return hipGetLastError();
+}
+
+hipError_t launch_state_copy(const double* const* src, double* const* dst, double* const* dst2, const DevMesh& M,
+                             unsigned long long* slots, int nslots, const int* err, int* report, hipStream_t s) {
+    StateCopy a;
+    const int n = M.n;
+    bool pairs = (n & 1) == 0 && dst && !dst2;
+    for (int k = 0; k < 5; ++k) {
+        a.src[k] = src[k];
+        a.dst[k] = dst ? dst[k] : nullptr;
+        a.dst2[k] = dst2 ? dst2[k] : nullptr;
+        pairs = pairs && (((uintptr_t)a.src[k] | (uintptr_t)a.dst[k]) & 15) == 0;
+    }
+    a.chunk_pid = M.chunk_pid;
+    a.seg_end = M.seg_end;
+    a.slots = slots;
+    a.nslots = nslots;
+    a.err = err;
+    a.report = report;
+    const int items = pairs ? n / 2 : n;
+    const int g = std::max(1, std::min(grid_cells(items, 256), 2048));
+    if (pairs) hipLaunchKernelGGL(k_state_copy<true>, dim3(g), dim3(256), 0, s, a, n);
+    else hipLaunchKernelGGL(k_state_copy<false>, dim3(g), dim3(256), 0, s, a, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_report(const double* dt, const int* err, double* dt_out, int* err_out, hipStream_t s) {
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, s, dt, err, dt_out, err_out);
     return hipGetLastError();
 }
 
