@@ -61,14 +61,15 @@ struct zfv3_ctx {
     int* d_type = nullptr;        // [6][n]
     int* d_adj = nullptr;         // [6][n]
     double* d_slot = nullptr;     // fcx, fcy, fcz, area, w: [5][6][n]
-    double* d_z[3] = {nullptr, nullptr, nullptr};   // three states of [6][n]
-    double* d_G = nullptr;        // [15][n]
+    double2* d_z[2] = {nullptr, nullptr};   // two states of [3][n]
+    double2* d_rec = nullptr;     // the predictor's records, [kRecPairs][n]
     int* d_wait[2] = {nullptr, nullptr};
     unsigned long long* d_slots = nullptr;   // three rotating CFL slots
     double* d_dt = nullptr;
     int* d_err = nullptr;
     double* d_part = nullptr;     // totals partial sums [5][blocks]
-    double* d_tab = nullptr;      // the Cuboid's geometry tables, when every cell matches them
+    double2* d_tab = nullptr;     // the Cuboid's geometry tables, when every cell matches them
+    double area1[6] = {}, vol1 = 0.0;
     int tab_bcode[6] = {0, 0, 0, 0, 0, 0};
     int tab_per[3] = {0, 0, 0};
     bool use_tables = true;
@@ -77,7 +78,7 @@ struct zfv3_ctx {
     bool configured = false, have_state = false, dt_valid = false;
     bool dt_ready = false;        // slot `cur` holds the CFL minimum of the current state
     zfv_smf_params prm{};
-    int zi = 0, hi = 1, ni = 2;   // init / half / next buffers
+    int zi = 0;                   // the current state's buffer; the other takes the next one
     int wi = 0, cur = 0;
     // kernel timing: an event pair around every launch while enabled
     struct Timed {
@@ -103,7 +104,7 @@ struct zfv3_ctx {
         for (void* p : allocs) (void)hipFree(p);
         allocs.clear();
         d_cell = nullptr; d_type = nullptr; d_adj = nullptr; d_slot = nullptr;
-        d_z[0] = d_z[1] = d_z[2] = nullptr; d_G = nullptr; d_wait[0] = d_wait[1] = nullptr;
+        d_z[0] = d_z[1] = nullptr; d_rec = nullptr; d_wait[0] = d_wait[1] = nullptr;
         d_slots = nullptr; d_dt = nullptr; d_err = nullptr; d_part = nullptr; d_tab = nullptr;
     }
     template <class T>
@@ -122,8 +123,10 @@ struct zfv3_ctx {
         if (d_tab) {
             M.tnx = nx; M.tny = ny; M.tnz = nz;
             M.tab = d_tab;
-            for (int k = 0; k < 6; ++k) M.bcode[k] = tab_bcode[k];
-            for (int a = 0; a < 3; ++a) M.per[a] = tab_per[a];
+            for (int k = 0; k < 6; ++k) M.area1[k] = area1[k];
+            M.vol1 = vol1;
+            for (int k = 0; k < 6; ++k) M.bcodes |= tab_bcode[k] << (4 * k);
+            for (int a = 0; a < 3; ++a) M.per |= tab_per[a] ? 1 << a : 0;
         }
         M.cx = d_cell; M.cy = d_cell + N; M.cz = d_cell + 2 * N; M.vol = d_cell + 3 * N; M.h = d_cell + 4 * N;
         M.type = d_type; M.adj = d_adj;
@@ -131,10 +134,10 @@ struct zfv3_ctx {
         return M;
     }
     Dev3State state(int k) const {
-        double* b = d_z[k];
-        const size_t N = (size_t)n;
-        return Dev3State{b, b + N, b + 2 * N, b + 3 * N, b + 4 * N, b + 5 * N};
+        return Dev3State{d_z[k], n};
     }
+    // rows of 6 n doubles in the buffer that the next step will write
+    double* staging() const { return (double*)d_z[zi ^ 1]; }
     Eos eos() const { return Eos{prm.gamma, prm.P0, prm.e0}; }
     unsigned long long* slot(int k) const { return d_slots + (size_t)k * kSlotWords; }
 };
@@ -257,33 +260,48 @@ void build_cuboid(zfv3_ctx* m, int nx, int ny, int nz, double xmin, double xmax,
 // The Cuboid's geometry as 1D tables (the layout of Dev3Mesh::tab): each
 // value taken from the first cell along its axis, then every cell and slot
 // compared with them bit for bit; false (no tables) on any difference.
-bool build_tables(const zfv3_ctx* m, std::vector<double>& tab, int bcode[6], int per[3]) {
+bool build_tables(const zfv3_ctx* m, std::vector<double2>& tab, double area[6], double* vol, int bcode[6],
+                  int per[3]) {
     const int nx = m->nx, ny = m->ny, nz = m->nz, L = nx + ny + nz;
     const int len[3] = {nx, ny, nz}, base[3] = {0, nx, nx + ny}, st[3] = {ny * nz, nz, 1};
-    tab.assign(tab3_size(nx, ny, nz), 0.0);
+    tab.assign(tab3_size(nx, ny, nz), make_double2(0.0, 0.0));
     auto slot = [](int c, int s) { return (size_t)kSides * c + s; };
     const std::vector<double>* fcs[3] = {&m->fcx, &m->fcy, &m->fcz};
     const std::vector<double>* ccs[3] = {&m->cx, &m->cy, &m->cz};
+    auto at = [&](int q, int a, int t, int up) -> double& {
+        double2& v = tab[(size_t)q * L + base[a] + t];
+        return up ? v.y : v.x;
+    };
+    for (int a = 0; a < 3; ++a) per[a] = m->bnd[slot((len[a] - 1) * st[a], 2 * a + 1)] == ZFV_PERIODIC;
+    for (int s = 0; s < kSides; ++s) {
+        const int b = s >> 1;
+        bcode[s] = slot_code(m->bnd[slot((s & 1) ? (len[b] - 1) * st[b] : 0, s)]);
+        area[s] = m->area[slot(0, s)];
+    }
+    *vol = m->vol[0];
     for (int a = 0; a < 3; ++a)
         for (int t = 0; t < len[a]; ++t) {
             const int c = t * st[a];
-            tab[18 * (size_t)L + base[a] + t] = (*ccs[a])[c];
-            for (int s = 0; s < kSides; ++s) tab[(size_t)(3 * s + a) * L + base[a] + t] = (*fcs[a])[slot(c, s)];
+            const double cc = (*ccs[a])[c];
+            for (int s = 0; s < kSides; ++s) {
+                const double fc = (*fcs[a])[slot(c, s)], off = fc - cc;
+                const int up = s & 1;
+                at(s >> 1, a, t, up) = off;
+                if ((s >> 1) != a) continue;
+                const double n = up ? 1.0 : -1.0;
+                const double d = 2.0 * ((fc - cc) * n), mirror = cc + d * n;   // symm_point (amr_faces.h:197-199)
+                const bool edge = up ? t == len[a] - 1 : t == 0;
+                const double across = edge ? mirror : (*ccs[a])[c + (up ? st[a] : -st[a])];
+                at(3, a, t, up) = edge && bcode[s] != SC_PERIODIC ? off : fc - across;
+                at(4, a, t, up) = across - cc;
+                at(5, a, t, up) = m->w[slot(c, s)];
+            }
         }
-    for (int s = 0; s < kSides; ++s) {
-        const int b = s >> 1;
-        for (int t = 0; t < len[b]; ++t) tab[19 * (size_t)L + (size_t)s * L + base[b] + t] = m->w[slot(t * st[b], s)];
-        tab[25 * (size_t)L + s] = m->area[slot(0, s)];
-        const int edge_cell = (s & 1) ? (len[b] - 1) * st[b] : 0;
-        bcode[s] = slot_code(m->bnd[slot(edge_cell, s)]);
-    }
-    tab[25 * (size_t)L + 6] = m->vol[0];
-    for (int a = 0; a < 3; ++a) per[a] = m->bnd[slot((len[a] - 1) * st[a], 2 * a + 1)] == ZFV_PERIODIC;
     for (int c = 0; c < m->n; ++c) {
         const int idx[3] = {c / st[0], (c % st[0]) / nz, c % nz};
-        if (m->vol[c] != tab[25 * (size_t)L + 6]) return false;
+        if (m->vol[c] != *vol) return false;
         for (int a = 0; a < 3; ++a)
-            if ((*ccs[a])[c] != tab[18 * (size_t)L + base[a] + idx[a]]) return false;
+            if ((*ccs[a])[c] != (*ccs[a])[(size_t)idx[a] * st[a]]) return false;
         for (int s = 0; s < kSides; ++s) {
             const int b = s >> 1, up = s & 1;
             const bool edge = up ? idx[b] == len[b] - 1 : idx[b] == 0;
@@ -292,10 +310,10 @@ bool build_tables(const zfv3_ctx* m, std::vector<double>& tab, int bcode[6], int
             int nb = up ? c + st[b] : c - st[b];
             if (edge) nb = per[b] ? (up ? c - (len[b] - 1) * st[b] : c + (len[b] - 1) * st[b]) : c;
             if (slot_code(m->bnd[o]) != code || m->adj[o] != nb) return false;
-            if (m->area[o] != tab[25 * (size_t)L + s]) return false;
-            if (m->w[o] != tab[19 * (size_t)L + (size_t)s * L + base[b] + idx[b]]) return false;
+            if (m->area[o] != area[s]) return false;
+            if (m->w[o] != at(5, b, idx[b], up)) return false;
             for (int a = 0; a < 3; ++a)
-                if ((*fcs[a])[o] != tab[(size_t)(3 * s + a) * L + base[a] + idx[a]]) return false;
+                if ((*fcs[a])[o] != (*fcs[a])[slot(idx[a] * st[a], s)]) return false;
         }
     }
     return true;
@@ -308,17 +326,17 @@ int upload_mesh(zfv3_ctx* ctx) {
     int r;
     if ((r = ctx->alloc(&ctx->d_cell, 5 * N)) || (r = ctx->alloc(&ctx->d_type, S)) ||
         (r = ctx->alloc(&ctx->d_adj, S)) || (r = ctx->alloc(&ctx->d_slot, 5 * S)) ||
-        (r = ctx->alloc(&ctx->d_z[0], 6 * N)) || (r = ctx->alloc(&ctx->d_z[1], 6 * N)) ||
-        (r = ctx->alloc(&ctx->d_z[2], 6 * N)) || (r = ctx->alloc(&ctx->d_G, 15 * N)) ||
+        (r = ctx->alloc(&ctx->d_z[0], 3 * N)) || (r = ctx->alloc(&ctx->d_z[1], 3 * N)) ||
+        (r = ctx->alloc(&ctx->d_rec, kRecPairs * N)) ||
         (r = ctx->alloc(&ctx->d_wait[0], N)) || (r = ctx->alloc(&ctx->d_wait[1], N)) ||
         (r = ctx->alloc(&ctx->d_slots, 3 * (size_t)kSlotWords)) || (r = ctx->alloc(&ctx->d_dt, 1)) || (r = ctx->alloc(&ctx->d_err, 1)))
         return r;
     ctx->blocks = (int)((N + 255) / 256);
     if ((r = ctx->alloc(&ctx->d_part, 5 * (size_t)ctx->blocks))) return r;
-    std::vector<double> tab;
-    if (ctx->use_tables && build_tables(ctx, tab, ctx->tab_bcode, ctx->tab_per)) {
+    std::vector<double2> tab;
+    if (ctx->use_tables && build_tables(ctx, tab, ctx->area1, &ctx->vol1, ctx->tab_bcode, ctx->tab_per)) {
         if ((r = ctx->alloc(&ctx->d_tab, tab.size()))) return r;
-        Z3HIP(hipMemcpy(ctx->d_tab, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
+        Z3HIP(hipMemcpy(ctx->d_tab, tab.data(), tab.size() * sizeof(double2), hipMemcpyHostToDevice));
     }
     // host staging in the device layout
     std::vector<double> cell(5 * N), slot(5 * S);
@@ -342,8 +360,8 @@ int upload_mesh(zfv3_ctx* ctx) {
     Z3HIP(hipMemset(ctx->d_err, 0, sizeof(int)));
     Z3HIP(hipMemset(ctx->d_wait[0], 0, N * sizeof(int)));
     Z3HIP(hipMemset(ctx->d_wait[1], 0, N * sizeof(int)));
-    Z3HIP(hipMemset(ctx->d_G, 0, 15 * N * sizeof(double)));
-    ctx->zi = 0; ctx->hi = 1; ctx->ni = 2; ctx->wi = 0; ctx->cur = 0;
+    Z3HIP(hipMemset(ctx->d_rec, 0, kRecPairs * N * sizeof(double2)));
+    ctx->zi = 0; ctx->wi = 0; ctx->cur = 0;
     ctx->have_state = false;
     ctx->dt_valid = false;
     ctx->dt_ready = false;
@@ -500,7 +518,8 @@ int zfv3_state_upload(zfv3_ctx* ctx, const double* rho, const double* u, const d
     const double* src[6] = {rho, u, v, w, p, e};
     Z3HIP(hipStreamSynchronize(ctx->stream));
     for (int k = 0; k < 6; ++k)
-        Z3HIP(hipMemcpy(ctx->d_z[ctx->zi] + k * N, src[k], N * sizeof(double), hipMemcpyHostToDevice));
+        Z3HIP(hipMemcpy(ctx->staging() + k * N, src[k], N * sizeof(double), hipMemcpyHostToDevice));
+    Z3HIP(launch3_pack(ctx->staging(), ctx->state(ctx->zi), ctx->stream));
     ctx->have_state = true;
     return state_changed(ctx);
 }
@@ -510,9 +529,10 @@ int zfv3_state_download(zfv3_ctx* ctx, double* rho, double* u, double* v, double
     if (r) return r;
     const size_t N = (size_t)ctx->n;
     double* dst[6] = {rho, u, v, w, p, e};
+    Z3HIP(launch3_rows(ctx->d_z[ctx->zi], ctx->n, 0, 6, ctx->staging(), ctx->stream));
     for (int k = 0; k < 6; ++k)
         if (dst[k])
-            Z3HIP(hipMemcpyAsync(dst[k], ctx->d_z[ctx->zi] + k * N, N * sizeof(double), hipMemcpyDeviceToHost,
+            Z3HIP(hipMemcpyAsync(dst[k], ctx->staging() + k * N, N * sizeof(double), hipMemcpyDeviceToHost,
                                  ctx->stream));
     return read_err(ctx);
 }
@@ -539,7 +559,12 @@ int zfv3_grad_download(zfv3_ctx* ctx, double* g) {
     int r = need_mesh(ctx);
     if (r) return r;
     if (!g) return fail(ZFV_ERR_ARG, "null gradient array");
-    Z3HIP(hipMemcpyAsync(g, ctx->d_G, 15 * (size_t)ctx->n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    const size_t row = 5 * (size_t)ctx->n;
+    double* buf = ctx->staging();
+    for (int a = 0; a < 3; ++a) {
+        Z3HIP(launch3_rows(ctx->d_rec, ctx->n, 6 + 5 * a, 5, buf, ctx->stream));
+        Z3HIP(hipMemcpyAsync(g + a * row, buf, row * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    }
     return read_err(ctx);
 }
 
@@ -583,7 +608,7 @@ int zfv3_smf_step(zfv3_ctx* ctx, int n_steps) {
     for (int it = 0; it < n_steps; ++it) {
         const Dev3Ctl ctl{ctx->slot(ctx->cur), ctx->slot((ctx->cur + 1) % 3), ctx->slot((ctx->cur + 2) % 3),
                           ctx->prm.cfl, ctx->prm.max_dt, ctx->d_dt, ctx->d_err};
-        const Dev3State z = ctx->state(ctx->zi), h = ctx->state(ctx->hi), nx = ctx->state(ctx->ni);
+        const Dev3State z = ctx->state(ctx->zi), nx = ctx->state(ctx->zi ^ 1);
         int* w0 = ctx->d_wait[ctx->wi];
         int* w1 = ctx->d_wait[ctx->wi ^ 1];
         if (!ctx->dt_ready && (r = timed_launch(ctx, "dt", [&] { return launch3_dt(M, z, eos, ctl.dtmin, s); })))
@@ -592,16 +617,14 @@ int zfv3_smf_step(zfv3_ctx* ctx, int n_steps) {
             if ((r = timed_launch(ctx, "flux1", [&] { return launch3_flux1(flux, M, z, nx, eos, ctl, s); }))) return r;
         } else {
             if ((r = timed_launch(ctx, "grad_pred",
-                                  [&] { return launch3_grad_pred(lim, M, z, ctx->d_G, h, w0, eos, ctl, s); })))
+                                  [&] { return launch3_grad_pred(lim, M, z, ctx->d_rec, w0, eos, ctl, s); })))
                 return r;
             if ((r = timed_launch(ctx, "corr",
-                                  [&] { return launch3_corr(flux, M, z, h, ctx->d_G, w0, w1, nx, eos, ctl, s); })))
+                                  [&] { return launch3_corr(flux, M, z, ctx->d_rec, w1, nx, eos, ctl, s); })))
                 return r;
             ctx->wi ^= 1;
         }
-        const int t = ctx->zi;
-        ctx->zi = ctx->ni;
-        ctx->ni = t;
+        ctx->zi ^= 1;
         ctx->cur = (ctx->cur + 1) % 3;
         ctx->dt_valid = true;
         ctx->dt_ready = true;

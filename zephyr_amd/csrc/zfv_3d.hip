@@ -229,17 +229,6 @@ __device__ __forceinline__ void to_global3(int s, Q3& f) {
     }
 }
 
-// boundary_value (sm_fluid.cpp:69-79): a wall reflects the velocity
-// component along the side's axis, v - 2 v.
-__device__ __forceinline__ Z3 wall3(int s, const Z3& z) {
-    Z3 r = z;
-    if (s < 2) r.u = z.u - 2.0 * z.u;
-    else if (s < 4) r.v = z.v - 2.0 * z.v;
-    else r.w = z.w - 2.0 * z.w;
-    return r;
-}
-
-__device__ __forceinline__ double axis_of(const double* v, int s) { return v[s >> 1]; }
 __device__ __forceinline__ double sgn_of(int s) { return (s & 1) ? 1.0 : -1.0; }
 
 // The five rows rho, u, v, w, p of a state.
@@ -255,10 +244,33 @@ __device__ __forceinline__ void zset(Z3& z, int k, double v) {
 }
 
 __device__ __forceinline__ Z3 load3(const Dev3State& s, int c) {
-    return Z3{s.r[c], s.u[c], s.v[c], s.w[c], s.p[c], s.e[c]};
+    const double2 a = s.q[c], b = s.q[(size_t)s.n + c], d = s.q[2 * (size_t)s.n + c];
+    return Z3{a.x, a.y, b.x, b.y, d.x, d.y};
 }
 __device__ __forceinline__ void store3(const Dev3State& s, int c, const Z3& z) {
-    s.r[c] = z.r; s.u[c] = z.u; s.v[c] = z.v; s.w[c] = z.w; s.p[c] = z.p; s.e[c] = z.e;
+    s.q[c] = make_double2(z.r, z.u);
+    s.q[(size_t)s.n + c] = make_double2(z.v, z.w);
+    s.q[2 * (size_t)s.n + c] = make_double2(z.p, z.e);
+}
+
+// What the predictor hands to the corrector (Dev3Mesh's record, kRecPairs
+// pairs a cell): the half state, the gradient of rho, u, v, w, p by field, and
+// the isolation counter.
+struct Rec3 {
+    Z3 h;
+    double g[3][5];
+    double wait;
+};
+__device__ __forceinline__ Rec3 rec_of(const double2* t) {
+    Rec3 r;
+    r.h = Z3{t[0].x, t[0].y, t[1].x, t[1].y, t[2].x, t[2].y};
+    const double2* g = t + 3;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int k = 0; k < 5; ++k) r.g[a][k] = ((5 * a + k) & 1) ? g[(5 * a + k) >> 1].y : g[(5 * a + k) >> 1].x;
+    r.wait = t[10].y;
+    return r;
 }
 
 // FaceExtraDirect (face_extra.h:135-149) on rho, u, v, w, p: du =
@@ -350,12 +362,13 @@ struct Geo3 {
     __device__ __forceinline__ int len(int a) const { return a == 0 ? M.tnx : (a == 1 ? M.tny : M.tnz); }
     __device__ __forceinline__ int base(int a) const { return a == 0 ? 0 : (a == 1 ? M.tnx : M.tnx + M.tny); }
     __device__ __forceinline__ int stride(int a) const { return a == 0 ? M.tny * M.tnz : (a == 1 ? M.tnz : 1); }
-    __device__ __forceinline__ double centre(int a) const {
-        if constexpr (TAB) return M.tab[18 * L + base(a) + idx(a)];
-        return a == 0 ? M.cx[c] : (a == 1 ? M.cy[c] : M.cz[c]);
+    // of row q, the value of the lower or the upper side
+    __device__ __forceinline__ double at(int q, int a, int up) const {
+        const double2 t = M.tab[q * L + base(a) + idx(a)];
+        return up ? t.y : t.x;
     }
     __device__ __forceinline__ double vol() const {
-        if constexpr (TAB) return M.tab[25 * L + 6];
+        if constexpr (TAB) return M.vol1;
         return M.vol[c];
     }
     __device__ __forceinline__ bool edge(int s) const {
@@ -363,40 +376,71 @@ struct Geo3 {
         return (s & 1) ? idx(a) == len(a) - 1 : idx(a) == 0;
     }
     __device__ __forceinline__ int type(int s) const {
-        if constexpr (TAB) return edge(s) ? M.bcode[s] : SC_INNER;
+        if constexpr (TAB) return edge(s) ? (M.bcodes >> (4 * s)) & 15 : SC_INNER;
         return M.type[s * M.stride + c];
     }
     __device__ __forceinline__ int adj(int s) const {
         if constexpr (TAB) {
             const int a = s >> 1, st = stride(a), up = s & 1;
             if (!edge(s)) return up ? c + st : c - st;
-            if (!M.per[a]) return c;
+            if (!((M.per >> a) & 1)) return c;
             return up ? c - (len(a) - 1) * st : c + (len(a) - 1) * st;
         }
         return M.adj[s * M.stride + c];
     }
-    __device__ __forceinline__ double fc(int s, int a) const {
-        if constexpr (TAB) return M.tab[(3 * s + a) * L + base(a) + idx(a)];
-        const int so = s * M.stride + c;
-        return a == 0 ? M.fcx[so] : (a == 1 ? M.fcy[so] : M.fcz[so]);
-    }
     __device__ __forceinline__ double area(int s) const {
-        if constexpr (TAB) return M.tab[25 * L + s];
+        if constexpr (TAB) return M.area1[s];
         return M.area[s * M.stride + c];
     }
     __device__ __forceinline__ double w(int s) const {
-        if constexpr (TAB) return M.tab[19 * L + s * L + base(s >> 1) + idx(s >> 1)];
+        if constexpr (TAB) return at(5, s >> 1, s & 1);
         return M.w[s * M.stride + c];
     }
-    // component a of the centre of the neighbour nb across inner side s
-    __device__ __forceinline__ double ncentre(int s, int nb, int a) const {
-        if constexpr (TAB) {
-            if (a != (s >> 1)) return centre(a);
-            return M.tab[18 * L + base(a) + idx(a) + ((s & 1) ? 1 : -1)];
-        }
-        return a == 0 ? M.cx[nb] : (a == 1 ? M.cy[nb] : M.cz[nb]);
+    // component a of the vector from the cell's centre to the centre of side s
+    __device__ __forceinline__ double off(int s, int a) const {
+        if constexpr (TAB) return at(s >> 1, a, s & 1);
+        return fc(s, a) - centre(a, c);
+    }
+    // the same from the centre across side s: the neighbour's, the mirror
+    // point of the cell's own on a periodic side, the cell's own on a boundary
+    __device__ __forceinline__ double noff(int s, int t, int nb, int a) const {
+        if constexpr (TAB) return at(a == (s >> 1) ? 3 : s >> 1, a, s & 1);
+        if (t == SC_INNER) return fc(s, a) - centre(a, nb);
+        if (t == SC_PERIODIC && a == (s >> 1)) return fc(s, a) - mirror(s);
+        return off(s, a);
+    }
+    // along the axis of side s: the neighbour's centre, or the mirror point
+    // on a boundary or a periodic side, less the cell's
+    __device__ __forceinline__ double dr(int s, int t, int nb) const {
+        if constexpr (TAB) return at(4, s >> 1, s & 1);
+        return (t == SC_INNER ? centre(s >> 1, nb) : mirror(s)) - centre(s >> 1, c);
+    }
+
+private:   // the slot arrays
+    __device__ __forceinline__ double centre(int a, int cell) const {
+        return a == 0 ? M.cx[cell] : (a == 1 ? M.cy[cell] : M.cz[cell]);
+    }
+    __device__ __forceinline__ double fc(int s, int a) const {
+        const int so = s * M.stride + c;
+        return a == 0 ? M.fcx[so] : (a == 1 ? M.fcy[so] : M.fcz[so]);
+    }
+    // symm_point: p + (2 (f - p).n) n
+    __device__ __forceinline__ double mirror(int s) const {
+        const int a = s >> 1;
+        const double d = 2.0 * ((fc(s, a) - centre(a, c)) * sgn_of(s));
+        return centre(a, c) + d * sgn_of(s);
     }
 };
+
+// boundary_value (sm_fluid.cpp:69-79) of the state read at geo.adj, which on a
+// boundary is the cell's own: a wall reflects the velocity component along
+// the side's axis, v - 2 v.
+__device__ __forceinline__ void reflect(int s, bool wall, Z3& z) {
+    const int a = s >> 1;
+    if (a == 0) z.u = wall ? z.u - 2.0 * z.u : z.u;
+    else if (a == 1) z.v = wall ? z.v - 2.0 * z.v : z.v;
+    else z.w = wall ? z.w - 2.0 * z.w : z.w;
+}
 
 }  // namespace
 
@@ -418,11 +462,8 @@ __device__ __forceinline__ double flux1_cell(const Dev3Mesh& M, const Dev3State&
     Q3 F{0.0, 0.0, 0.0, 0.0, 0.0};
     bool bad = false;
     for (int s = 0; s < 6; ++s) {
-        const int so = s * M.stride + c;
-        const int t = geo.type(s);
-        Z3 zn = zc;
-        if (t == SC_INNER || t == SC_PERIODIC) zn = load3(in, geo.adj(s));
-        else if (t == SC_WALL) zn = wall3(s, zc);
+        Z3 zn = load3(in, geo.adj(s));
+        reflect(s, geo.type(s) == SC_WALL, zn);
         Z3 lm = zc, lp = zn;
         to_local3(s, lm);
         to_local3(s, lp);
@@ -459,49 +500,30 @@ __global__ void __launch_bounds__(256) k3_flux1(Dev3Mesh M, Dev3State in, Dev3St
 
 // SmFluid::compute_grad (gradient::LSM, gradient.h:226-282, then
 // gradient::limiting, gradient.h:412-474) fused with fluxes_stage1
-// (sm_fluid.cpp:176-253).  G: [3][5][stride], d/dx, d/dy, d/dz of rho, u,
-// v, w, p.
+// (sm_fluid.cpp:176-253) into the records.  The system is diagonal, so the axes are taken one after the
+// other, each with only its own two neighbours in registers and its derivatives
+// stored at once: 129 registers for 190, 96^3 cells with MC 91 -> 69 us, of which
+// the vector instructions take 55.
 template <int LIM, bool TAB>
-__global__ void __launch_bounds__(256) k3_grad_pred(Dev3Mesh M, Dev3State in, double* __restrict__ G, Dev3State half,
+__global__ void __launch_bounds__(256) k3_grad_pred(Dev3Mesh M, Dev3State in, double2* __restrict__ R,
                                                     const int* __restrict__ wait, Eos eos, Dev3Ctl ctl) {
     const int c = cell_of_thread();
     const double dt = block_dt(ctl);
     if (c >= M.n) return;
     const Geo3<TAB> geo(M, c);
     const Z3 zc = load3(in, c);
-    const double cc[3] = {geo.centre(0), geo.centre(1), geo.centre(2)};
-    // per slot: dr along its axis (zero across), the state across it
-    double dra[6], w[6];
-    Z3 zn[6];
+    int ts[6], nbs[6];
+    double dra[6], w[6], A[3];
 #pragma unroll
     for (int s = 0; s < 6; ++s) {
-        const int so = s * M.stride + c;
-        const int t = geo.type(s);
-        const int nb = geo.adj(s);
+        ts[s] = geo.type(s);
+        nbs[s] = geo.adj(s);
         w[s] = geo.w(s);
-        zn[s] = (t == SC_INNER || t == SC_PERIODIC) ? load3(in, nb) : (t == SC_WALL ? wall3(s, zc) : zc);
-        const double fc[3] = {geo.fc(s, 0), geo.fc(s, 1), geo.fc(s, 2)};
-        const double na = sgn_of(s);
-        if (t == SC_INNER) {
-            const double nc[3] = {geo.ncentre(s, nb, 0), geo.ncentre(s, nb, 1), geo.ncentre(s, nb, 2)};
-            dra[s] = axis_of(nc, s) - axis_of(cc, s);
-        } else {   // symm_point: p + (2 (f - p).n) n
-            const double d = 2.0 * ((axis_of(fc, s) - axis_of(cc, s)) * na);
-            dra[s] = (axis_of(cc, s) + d * na) - axis_of(cc, s);
-        }
+        dra[s] = geo.dr(s, ts[s], nbs[s]);   // (dr.n) n has the same component: n is a unit axis
     }
-    // A (diagonal) and F: sums over the slots in slot order
-    double A[3] = {0.0, 0.0, 0.0};
-    double F[3][5] = {};
 #pragma unroll
-    for (int s = 0; s < 6; ++s) {
-        const int a = s >> 1;
-        const double na = sgn_of(s);
-        const double drn = (dra[s] * na) * na;
-        A[a] = A[a] + (w[s] * drn) * dra[s];
-#pragma unroll
-        for (int k = 0; k < 5; ++k) F[a][k] = F[a][k] + (w[s] * (zk(zn[s], k) - zk(zc, k))) * drn;
-    }
+    for (int a = 0; a < 3; ++a)
+        A[a] = (w[2 * a] * dra[2 * a]) * dra[2 * a] + (w[2 * a + 1] * dra[2 * a + 1]) * dra[2 * a + 1];
     if (fabs(A[2]) < 1e-8) {
         A[2] = 1.0;
         if (fabs(A[1]) < 1e-8) A[1] = 1.0;
@@ -511,38 +533,41 @@ __global__ void __launch_bounds__(256) k3_grad_pred(Dev3Mesh M, Dev3State in, do
     const double B[3] = {c00 * invdet, c11 * invdet, c22 * invdet};
     double g[3][5];
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int k = 0; k < 5; ++k) g[a][k] = B[a] * F[a][k];
-    // limiting: limiter(2 du_n - dF, dF) dF, re-solved with the same A
-    double L[3][5] = {};
-#pragma unroll
-    for (int s = 0; s < 6; ++s) {
-        const int a = s >> 1;
-        const double na = sgn_of(s);
-        const double drn = (dra[s] * na) * na;
+    for (int a = 0; a < 3; ++a) {
+        const int lo = 2 * a, hi = 2 * a + 1;
+        Z3 zl = load3(in, nbs[lo]), zr = load3(in, nbs[hi]);
+        reflect(lo, ts[lo] == SC_WALL, zl);
+        reflect(hi, ts[hi] == SC_WALL, zr);
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
-            const double dF = zk(zn[s], k) - zk(zc, k);
-            const double du_n = g[a][k] * dra[s];
-            const double lim = limiter2<LIM>(2.0 * du_n - dF, dF) * dF;
-            L[a][k] = L[a][k] + (w[s] * lim) * drn;
+            const double dl = zk(zl, k) - zk(zc, k), dh = zk(zr, k) - zk(zc, k);
+            const double gk = B[a] * ((w[lo] * dl) * dra[lo] + (w[hi] * dh) * dra[hi]);
+            // limiting: limiter(2 du_n - dF, dF) dF, re-solved with the same A
+            const double ml = limiter2<LIM>(2.0 * (gk * dra[lo]) - dl, dl) * dl;
+            const double mh = limiter2<LIM>(2.0 * (gk * dra[hi]) - dh, dh) * dh;
+            g[a][k] = B[a] * ((w[lo] * ml) * dra[lo] + (w[hi] * mh) * dra[hi]);
+        }
+        // the record's pairs that are complete: doubles 6 + 5 a to 10 + 5 a
+        const size_t n = (size_t)M.stride;
+        double2* r = R + (a == 0 ? 3 : (a == 1 ? 5 : 8)) * n + c;
+        if (a == 1) {
+            r[0] = make_double2(g[0][4], g[1][0]);
+            r[n] = make_double2(g[1][1], g[1][2]);
+            r[2 * n] = make_double2(g[1][3], g[1][4]);
+        } else {
+            r[0] = make_double2(g[a][0], g[a][1]);
+            r[n] = make_double2(g[a][2], g[a][3]);
         }
     }
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-        for (int k = 0; k < 5; ++k) {
-            g[a][k] = B[a] * L[a][k];
-            G[(size_t)(a * 5 + k) * M.stride + c] = g[a][k];
-        }
+    const int wc = wait[c];
+    R[10 * (size_t)M.stride + c] = make_double2(g[2][4], (double)wc);
     // predictor
     Z3 zh = zc;
-    if (wait[c] <= 0) {
+    if (wc <= 0) {
         Q3 Fl{0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
         for (int s = 0; s < 6; ++s) {
-            const int so = s * M.stride + c;
-            Z3 zm = extrap3(zc, g, geo.fc(s, 0) - cc[0], geo.fc(s, 1) - cc[1], geo.fc(s, 2) - cc[2], eos);
+            Z3 zm = extrap3(zc, g, geo.off(s, 0), geo.off(s, 1), geo.off(s, 2), eos);
             if (is_bad3(zm, eos)) zm = zc;
             to_local3(s, zm);
             Q3 f = phys_flux3(zm);
@@ -564,77 +589,58 @@ __global__ void __launch_bounds__(256) k3_grad_pred(Dev3Mesh M, Dev3State in, do
         zh = to_z3(q, eos);
         if (is_bad3(zh, eos)) zh = zc;
     }
-    store3(half, c, zh);
+    store3(Dev3State{R, M.stride}, c, zh);
 }
 
 // SmFluid::fluxes_stage2, corrector (sm_fluid.cpp:255-366): wait read from
-// the pre-pass array, written to the other; returns the next step's CFL
-// candidate of the new state.
+// the record, written to the array of the next step; returns the next step's
+// CFL candidate of the new state.  The workgroup's cells leave their records in
+// LDS for the neighbours among them (all but a few along z, and along y while
+// nz < 256): with every neighbour read from memory the L1 cache was busy 89 % of
+// the time.  Three waves a SIMD, which spills two registers, since a wave waits
+// for loads 43 % of its time.  96^3 cells, HLLC: 165 us with one array a field
+// and no LDS, 137 with pairs, 119 so (133 at two waves); the vector instructions
+// alone take 87.  Evaluating each face once for both of its cells (tiles marched
+// along x) took 170: with 3D's larger state the exchange costs what it saves.
 template <int FLUX, bool TAB>
-__device__ __forceinline__ double corr_cell(const Dev3Mesh& M, const Dev3State& init, const Dev3State& half,
-                                            const double* __restrict__ G, const int* __restrict__ wait_in,
+__device__ __forceinline__ double corr_cell(const Dev3Mesh& M, const Dev3State& init, const double2* __restrict__ R,
                                             int* __restrict__ wait_out, const Dev3State& next, const Eos& eos,
-                                            const Dev3Ctl& ctl, double dt, int c) {
+                                            const Dev3Ctl& ctl, double dt, int c, bool live) {
+    __shared__ double2 recs[kRecPairs][256];
     const Geo3<TAB> geo(M, c);
-    const Z3 zc = load3(init, c);
-    const Z3 zch = load3(half, c);
-    const double cc[3] = {geo.centre(0), geo.centre(1), geo.centre(2)};
-    const int wc = wait_in[c];
-    double g[3][5];
+    double2 own[kRecPairs];
 #pragma unroll
-    for (int a = 0; a < 3; ++a)
+    for (int m = 0; m < kRecPairs; ++m) own[m] = R[(size_t)m * M.stride + c];
 #pragma unroll
-        for (int k = 0; k < 5; ++k) g[a][k] = G[(size_t)(a * 5 + k) * M.stride + c];
-    // the six slots' codes, neighbours and neighbours' counters first: one
-    // round trip for all of them instead of two per face
-    int ts[6], nbs[6];
-#pragma unroll
-    for (int s = 0; s < 6; ++s) {
-        ts[s] = geo.type(s);
-        nbs[s] = geo.adj(s);
-    }
-    bool rob[6];
-#pragma unroll
-    for (int s = 0; s < 6; ++s) rob[s] = wc > 0 || wait_in[nbs[s]] > 0;
+    for (int m = 0; m < kRecPairs; ++m) recs[m][threadIdx.x] = own[m];
+    __syncthreads();
+    if (!live) return INFINITY;
+    const Rec3 rc = rec_of(own);
+    const int c0 = c - (int)threadIdx.x;
     Q3 F{0.0, 0.0, 0.0, 0.0, 0.0};
     bool bad = false;
 #pragma unroll
     for (int s = 0; s < 6; ++s) {
-        const int so = s * M.stride + c;
-        const int t = ts[s];
-        const int nb = nbs[s];
-        const bool bound = t >= SC_WALL;
-        const double fc[3] = {geo.fc(s, 0), geo.fc(s, 1), geo.fc(s, 2)};
-        const Z3 znh = bound ? (t == SC_WALL ? wall3(s, zch) : zch) : load3(half, nb);
-        const bool robust = rob[s];
-        Z3 zm, zp;
-        if (robust) {
-            zm = zch;
-            zp = znh;
+        const int t = geo.type(s), nb = geo.adj(s), q = nb - c0;
+        double2 other[kRecPairs];
+        if ((unsigned)q < 256u) {
+#pragma unroll
+            for (int m = 0; m < kRecPairs; ++m) other[m] = recs[m][q];
         } else {
-            double nc[3];
-            if (t == SC_INNER) {
-                nc[0] = geo.ncentre(s, nb, 0); nc[1] = geo.ncentre(s, nb, 1); nc[2] = geo.ncentre(s, nb, 2);
-            } else {   // the mirror point of the cell centre
-                const double na = sgn_of(s);
-                const double d = 2.0 * ((axis_of(fc, s) - axis_of(cc, s)) * na);
-                nc[0] = cc[0]; nc[1] = cc[1]; nc[2] = cc[2];
-                nc[s >> 1] = axis_of(cc, s) + d * na;
-            }
-            zm = extrap3(zch, g, fc[0] - cc[0], fc[1] - cc[1], fc[2] - cc[2], eos);
-            if (is_bad3(zm, eos)) zm = zch;
-            if (!bound) {
-                double gn[3][5];
 #pragma unroll
-                for (int a = 0; a < 3; ++a)
-#pragma unroll
-                    for (int k = 0; k < 5; ++k) gn[a][k] = G[(size_t)(a * 5 + k) * M.stride + nb];
-                zp = extrap3(znh, gn, fc[0] - nc[0], fc[1] - nc[1], fc[2] - nc[2], eos);
-                if (is_bad3(zp, eos)) zp = znh;
-            } else {
-                zp = t == SC_WALL ? wall3(s, zm) : zm;
-            }
+            for (int m = 0; m < kRecPairs; ++m) other[m] = R[(size_t)m * M.stride + nb];
         }
+        const Rec3 rn = rec_of(other);
+        Z3 zm = rc.h, zp = rn.h;
+        const bool robust = rc.wait > 0.0 || rn.wait > 0.0;
+        if (!robust) {
+            zm = extrap3(rc.h, rc.g, geo.off(s, 0), geo.off(s, 1), geo.off(s, 2), eos);
+            if (is_bad3(zm, eos)) zm = rc.h;
+            zp = extrap3(rn.h, rn.g, geo.noff(s, t, nb, 0), geo.noff(s, t, nb, 1), geo.noff(s, t, nb, 2), eos);
+            if (is_bad3(zp, eos)) zp = rn.h;
+        }
+        // on a boundary nb is the cell itself, and zp so far is zm
+        reflect(s, t == SC_WALL, zp);
         to_local3(s, zm);
         to_local3(s, zp);
         Q3 f = robust ? hll3(zm, zp, eos, bad) : num_flux3<FLUX>(zm, zp, eos, bad);
@@ -646,6 +652,7 @@ __device__ __forceinline__ double corr_cell(const Dev3Mesh& M, const Dev3State& 
         F.mz = F.mz + f.mz * a;
         F.E = F.E + f.E * a;
     }
+    const Z3 zc = load3(init, c);
     Q3 q = to_q3(zc);
     const double coef = dt / geo.vol();
     q.r = q.r - coef * F.r;
@@ -654,6 +661,7 @@ __device__ __forceinline__ double corr_cell(const Dev3Mesh& M, const Dev3State& 
     q.mz = q.mz - coef * F.mz;
     q.E = q.E - coef * F.E;
     Z3 zn = to_z3(q, eos);
+    const int wc = (int)rc.wait;
     int wn;
     if (is_bad3(zn, eos)) {
         zn = zc;
@@ -668,15 +676,34 @@ __device__ __forceinline__ double corr_cell(const Dev3Mesh& M, const Dev3State& 
 }
 
 template <int FLUX, bool TAB>
-__global__ void __launch_bounds__(256) k3_corr(Dev3Mesh M, Dev3State init, Dev3State half, const double* __restrict__ G,
-                                               const int* __restrict__ wait_in, int* __restrict__ wait_out,
-                                               Dev3State next, Eos eos, Dev3Ctl ctl) {
+__global__ void __launch_bounds__(256, 3) k3_corr(Dev3Mesh M, Dev3State init, const double2* __restrict__ R,
+                                               int* __restrict__ wait_out, Dev3State next, Eos eos, Dev3Ctl ctl) {
     const int c = cell_of_thread();
     const double dt = block_dt(ctl);
     step_epilogue0(ctl, dt);
+    // past the end: the last workgroup's idle threads read cell n - 1
     const double cand =
-        c < M.n ? corr_cell<FLUX, TAB>(M, init, half, G, wait_in, wait_out, next, eos, ctl, dt, c) : INFINITY;
+        corr_cell<FLUX, TAB>(M, init, R, wait_out, next, eos, ctl, dt, c < M.n ? c : M.n - 1, c < M.n);
     block_min(ctl.next, cand);
+}
+
+// Double m0 + k of every cell, k < count, out of arrays of pairs as rows [k][n].
+__global__ void __launch_bounds__(256) k3_rows(const double2* __restrict__ q, int n, int m0, int count,
+                                               double* __restrict__ out) {
+    const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (c >= n) return;
+    const double* v = (const double*)q;
+    for (int k = 0; k < count; ++k) {
+        const int m = m0 + k;
+        out[(size_t)k * n + c] = v[2 * ((size_t)(m >> 1) * n + c) + (m & 1)];
+    }
+}
+
+// Rows rho, u, v, w, p, e into a state.
+__global__ void __launch_bounds__(256) k3_pack(const double* __restrict__ in, Dev3State z) {
+    const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const size_t n = (size_t)z.n;
+    if (c < z.n) store3(z, c, Z3{in[c], in[n + c], in[2 * n + c], in[3 * n + c], in[4 * n + c], in[5 * n + c]});
 }
 
 // Per-workgroup partial sums of V q: mass, momentum x, y, z, energy.
@@ -731,12 +758,11 @@ hipError_t launch3_flux1(int flux, const Dev3Mesh& M, const Dev3State& in, const
     return hipGetLastError();
 }
 
-hipError_t launch3_grad_pred(int limiter, const Dev3Mesh& M, const Dev3State& in, double* G, const Dev3State& half,
-                             const int* wait, const Eos& eos, const Dev3Ctl& ctl, hipStream_t s) {
+hipError_t launch3_grad_pred(int limiter, const Dev3Mesh& M, const Dev3State& in, double2* R, const int* wait, const Eos& eos, const Dev3Ctl& ctl, hipStream_t s) {
     const bool tab = M.tnx > 0;
 #define ZFV3_GP(L)                                                                                          \
-    if (tab) hipLaunchKernelGGL((k3_grad_pred<L, true>), g256(M.n), dim3(256), 0, s, M, in, G, half, wait, eos, ctl); \
-    else hipLaunchKernelGGL((k3_grad_pred<L, false>), g256(M.n), dim3(256), 0, s, M, in, G, half, wait, eos, ctl)
+    if (tab) hipLaunchKernelGGL((k3_grad_pred<L, true>), g256(M.n), dim3(256), 0, s, M, in, R, wait, eos, ctl); \
+    else hipLaunchKernelGGL((k3_grad_pred<L, false>), g256(M.n), dim3(256), 0, s, M, in, R, wait, eos, ctl)
     switch (limiter) {
         case 0: ZFV3_GP(0); break;
         case 1: ZFV3_GP(1); break;
@@ -756,15 +782,12 @@ hipError_t launch3_grad_pred(int limiter, const Dev3Mesh& M, const Dev3State& in
     return hipGetLastError();
 }
 
-hipError_t launch3_corr(int flux, const Dev3Mesh& M, const Dev3State& init, const Dev3State& half, const double* G,
-                        const int* wait_in, int* wait_out, const Dev3State& next, const Eos& eos, const Dev3Ctl& ctl,
-                        hipStream_t s) {
+hipError_t launch3_corr(int flux, const Dev3Mesh& M, const Dev3State& init, const double2* R, int* wait_out,
+                        const Dev3State& next, const Eos& eos, const Dev3Ctl& ctl, hipStream_t s) {
     const bool tab = M.tnx > 0;
 #define ZFV3_C(F)                                                                                               \
-    if (tab) hipLaunchKernelGGL((k3_corr<F, true>), g256(M.n), dim3(256), 0, s, M, init, half, G, wait_in, wait_out, \
-                                next, eos, ctl);                                                                  \
-    else hipLaunchKernelGGL((k3_corr<F, false>), g256(M.n), dim3(256), 0, s, M, init, half, G, wait_in, wait_out,  \
-                            next, eos, ctl)
+    if (tab) hipLaunchKernelGGL((k3_corr<F, true>), g256(M.n), dim3(256), 0, s, M, init, R, wait_out, next, eos, ctl); \
+    else hipLaunchKernelGGL((k3_corr<F, false>), g256(M.n), dim3(256), 0, s, M, init, R, wait_out, next, eos, ctl)
     switch (flux) {
         case 0: ZFV3_C(0); break;
         case 1: ZFV3_C(1); break;
@@ -776,6 +799,16 @@ hipError_t launch3_corr(int flux, const Dev3Mesh& M, const Dev3State& init, cons
         default: ZFV3_C(3); break;
     }
 #undef ZFV3_C
+    return hipGetLastError();
+}
+
+hipError_t launch3_rows(const double2* q, int n, int m0, int count, double* out, hipStream_t s) {
+    hipLaunchKernelGGL(k3_rows, g256(n), dim3(256), 0, s, q, n, m0, count, out);
+    return hipGetLastError();
+}
+
+hipError_t launch3_pack(const double* in, const Dev3State& z, hipStream_t s) {
+    hipLaunchKernelGGL(k3_pack, g256(z.n), dim3(256), 0, s, in, z);
     return hipGetLastError();
 }
 
