@@ -119,16 +119,35 @@ __device__ __forceinline__ void flux_hllc_pair(const Z& A, const Z& B, const Eos
     }
 }
 
+// HLL and Rusanov evaluated once.  From B's side the bounds are A's negated and
+// exchanged, so each sum holds the same products, as x - y for y - x: its
+// rounded value is A's, negated, and GB = FA.  Not so where a wave speed is
+// NaN (`odd` above); there B's side is evaluated.
+template <int FLUX>
+__device__ __forceinline__ void flux_even_pair(const Z& A, const Z& B, const Eos& eos, bool& nanA, bool& nanB, Q& FA,
+                                               Q& GB) {
+    const double cA = eos_c(eos, A.r, A.p), cB = eos_c(eos, B.r, B.p);
+    const bool odd = __builtin_isunordered(A.u - cA, B.u - cB) | __builtin_isunordered(A.u + cA, B.u + cB);
+    FA = num_flux<FLUX>(A, B, eos, nanA);
+    GB = FA;
+    nanB = nanA;
+    if (__builtin_expect(__any(odd), 0)) {
+        bool n = false;
+        const Q g = mirrored(num_flux<FLUX>(mirrored(B), mirrored(A), eos, n));
+        if (odd) {
+            GB = g;
+            nanB = n;
+        }
+    }
+}
+
 template <int FLUX>
 __device__ __forceinline__ void flux_pair(const Z& A, const Z& B, const Eos& eos, bool& nanA, bool& nanB, Q& FA,
                                           Q& GB) {
+    static_assert(FLUX >= 1 && FLUX <= 3, "Rusanov, HLL, HLLC");
     nanA = nanB = false;
-    if constexpr (FLUX == 3) {
-        flux_hllc_pair(A, B, eos, nanA, nanB, FA, GB);
-    } else {
-        FA = num_flux<FLUX>(A, B, eos, nanA);
-        GB = mirrored(num_flux<FLUX>(mirrored(B), mirrored(A), eos, nanB));
-    }
+    if constexpr (FLUX == 3) flux_hllc_pair(A, B, eos, nanA, nanB, FA, GB);
+    else flux_even_pair<FLUX>(A, B, eos, nanA, nanB, FA, GB);
 }
 
 // The same with the isolation mode's HLL flux on `robust` lanes.
