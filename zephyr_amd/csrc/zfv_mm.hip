@@ -276,31 +276,32 @@ __global__ void __launch_bounds__(kBlock) k_mm_crp_mark(DevMesh M, MmLayer in, M
     if (any && cells) cells[atomicAdd(count + 1, 1u)] = c;
 }
 
-// The composite Riemann flux of each listed face, one face per thread: the
-// face-frame states, the master material
-// (master_component, mm_fluid.cpp:201-226), the PLIC face fraction of the
-// upwind cell's interface (alpha_sigma, :241-254, with the normals of
-// interface_recovery) and calc_crp_flux (:259-337), rotated to the global
-// frame, into CF[slot][k][stride].  These faces are few and need many more
-// registers than the plain HLLC faces of k_mm_flux1, hence the compaction.
+// The composite Riemann flux of each listed face, two lanes a face: the
+// face-frame states, the master material (master_component,
+// mm_fluid.cpp:201-226), the PLIC face fraction of the upwind cell's interface
+// (alpha_sigma, :241-254, with the normals of interface_recovery) and
+// calc_crp_flux (:259-337) in two parts, rotated to the global frame, into
+// CF[slot][k][stride].  These faces are few and need many more registers than
+// the plain HLLC faces of k_mm_flux1, hence the compaction; what bounds the
+// kernel is one face's chain of divisions and closures, and the paths that the
+// lanes of a wavefront do not share.  With calc_crp_part's selected inputs they
+// share nearly all, so wavefronts are full (2748 faces of 384^2 cells, first
+// order: 46 us with the reference's branches, four faces a wavefront; 34, 32, 28,
+// 24, 23 us with 2, 4, 8, 16 and 32).
 template <int NM, int ACC>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) k_mm_crp(DevMesh M, MmLayer in, MmLayer half, const double* __restrict__ gx,
-                                            const double* __restrict__ gy, Mix mx, StepCtl ctl, MmOpts opt,
+__global__ void __launch_bounds__(64) k_mm_crp(DevMesh M, MmLayer in, MmLayer half,
+                                               const double* __restrict__ gx,
+                                               const double* __restrict__ gy, Mix mx, StepCtl ctl, MmOpts opt,
                                             const double* __restrict__ inx, const double* __restrict__ iny,
                                             const int* __restrict__ list, const unsigned int* count,
                                             double* __restrict__ CF) {
     constexpr int K = 4 + NM;
     const int st = M.stride;
     const int n_faces = (int)*count;
-    // L active lanes per one-wavefront workgroup: the faces' branchy paths
-    // (closures, wave configurations) diverge, and a wavefront executes the
-    // union of its lanes' paths, so few faces are spread over many
-    // wavefronts; a long list fills whole wavefronts.
-    int L = 4;
-    while (L < 64 && (long long)L * gridDim.x < n_faces) L <<= 1;
-    const int lane = (int)threadIdx.x;
+    const bool role_a = (threadIdx.x & 1) == 0;
     bool bad = false;
-    for (int e = (int)blockIdx.x * L + lane; lane < L && e < n_faces; e += (int)gridDim.x * L) {
+    // a face's two lanes leave together, so both are there for the exchange
+    for (int e = (int)blockIdx.x * 32 + ((int)threadIdx.x >> 1); e < n_faces; e += (int)gridDim.x * 32) {
         const int so = list[e];
         const int s = so / st, c = so - s * st;
         const double dt = opt.dt_scale * step_dt(ctl, 0);
@@ -337,7 +338,14 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
                   : opt.crp == 2 ? face_fraction_v5(a_L, a_R) : face_fraction_s(a_L, a_R);
         }
         double F[K];
-        calc_crp_flux<NM>(zm, zp, h_L, h_R, iA, a_sig, dt, mx, F, bad);
+        const bool two = calc_crp_part<NM>(zm, zp, h_L, h_R, iA, a_sig, dt, mx, role_a, F, bad);
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const double o = __shfl_xor(F[k], 1, 64);
+            const double fA = role_a ? F[k] : o, fB = role_a ? o : F[k];
+            F[k] = two ? a_sig * fA + (1.0 - a_sig) * fB : F[k];
+        }
+        if (!role_a) continue;
         const Q g = frame_global(fr, Q{F[0], F[1], F[2], F[3]});
         F[1] = g.mx;
         F[2] = g.my;

@@ -747,23 +747,6 @@ __device__ __forceinline__ void crp_classic(const MZ<NM>& zLA, const MZ<NM>& zLB
     }
 }
 
-// CrpFlux::inverse (crp_flux.cpp:493-512): the classic problem mirrored in x
-// (PState::inverse flips u, Flux::inverse negates all but m_x, models.cpp:219-221, 506-515).
-template <int NM>
-__device__ __forceinline__ void crp_inverse(const MZ<NM>& zLA, const MZ<NM>& zRA, const MZ<NM>& zRB, const Mix& mx, double delta,
-                            double dt, double* out, bool& err) {
-    MZ<NM> a = zRB, b = zRA, c = zLA;
-    a.u = -a.u;
-    b.u = -b.u;
-    c.u = -c.u;
-    crp_classic<NM>(a, b, c, mx, delta, dt, out, err);
-    out[0] = -out[0];
-    out[2] = -out[2];
-    out[3] = -out[3];
-#pragma unroll
-    for (int i = 0; i < NM; ++i) out[4 + i] = -out[4 + i];
-}
-
 __device__ __forceinline__ double sg_energy_rT(const Mat& m, double rho, double T) {   // stiffened_gas.cpp:131-138
     return m.e0 + m.Cv * (T - m.T0) + m.P0 / rho;
 }
@@ -856,50 +839,74 @@ __device__ __forceinline__ int master_component(const MZ<NM>& zm, const MZ<NM>& 
     return master;
 }
 
-// MmFluid::calc_crp_flux (mm_fluid.cpp:259-337).
 template <int NM>
-__device__ __forceinline__ void calc_crp_flux(const MZ<NM>& zL, const MZ<NM>& zR, double hL, double hR, int iA, double a_sig,
-                              double dt, const Mix& mx, double* F, bool& err) {
-    constexpr int K = 4 + NM;
-    const double aL = alpha_of<NM>(zL, iA), aR = alpha_of<NM>(zR, iA);
-    if ((aL == 0.0 || aL == 1.0) && (aR == 0.0 || aR == 1.0)) {
-        hllc_mm<NM>(zL, zR, F, err);
-        return;
-    }
-    const double delta_L = (aL < a_sig ? aL / a_sig : (1.0 - aL) / (1.0 - a_sig)) * hL;
-    const double delta_R = (aR < a_sig ? aR / a_sig : (1.0 - aR) / (1.0 - a_sig)) * hR;
-    double fA[K], fB[K];
-    MZ<NM> xA, xB;
-    if (aL == 0.0) {
-        m_split<NM>(zR, mx, iA, xA, xB);
-        hllc_mm<NM>(zL, xA, fA, err);
-        crp_inverse<NM>(zL, xB, xA, mx, delta_R, dt, fB, err);
-    } else if (aL == 1.0) {
-        m_split<NM>(zR, mx, iA, xA, xB);
-        crp_inverse<NM>(zL, xA, xB, mx, delta_R, dt, fA, err);
-        hllc_mm<NM>(zL, xB, fB, err);
-    } else if (aR == 0.0) {
-        m_split<NM>(zL, mx, iA, xA, xB);
-        hllc_mm<NM>(xA, zR, fA, err);
-        crp_classic<NM>(xA, xB, zR, mx, delta_L, dt, fB, err);
-    } else if (aR == 1.0) {
-        m_split<NM>(zL, mx, iA, xA, xB);
-        crp_classic<NM>(xB, xA, zR, mx, delta_L, dt, fA, err);
-        hllc_mm<NM>(xB, zR, fB, err);
-    } else {
-        MZ<NM> yA, yB;
-        m_split<NM>(zL, mx, iA, xA, xB);
-        m_split<NM>(zR, mx, iA, yA, yB);
-        if (aL < aR) {
-            crp_classic<NM>(xB, xA, yA, mx, delta_L, dt, fA, err);
-            crp_inverse<NM>(xB, yB, yA, mx, delta_R, dt, fB, err);
-        } else {
-            crp_inverse<NM>(xA, yA, yB, mx, delta_R, dt, fA, err);
-            crp_classic<NM>(xA, xB, yB, mx, delta_L, dt, fB, err);
-        }
-    }
+__device__ __forceinline__ MZ<NM> select_mz(bool first, const MZ<NM>& a, const MZ<NM>& b) {
+    MZ<NM> r;
+    r.r = first ? a.r : b.r;
+    r.u = first ? a.u : b.u;
+    r.v = first ? a.v : b.v;
+    r.P = first ? a.P : b.P;
+    r.e = first ? a.e : b.e;
+    r.T = first ? a.T : b.T;
+    r.c = first ? a.c : b.c;
 #pragma unroll
-    for (int k = 0; k < K; ++k) F[k] = a_sig * fA[k] + (1.0 - a_sig) * fB[k];
+    for (int i = 0; i < NM; ++i) {
+        r.b[i] = first ? a.b[i] : b.b[i];
+        r.rh[i] = first ? a.rh[i] : b.rh[i];
+    }
+    return r;
+}
+
+// MmFluid::calc_crp_flux (mm_fluid.cpp:259-337) by two lanes of a face: the flux
+// of the master material's part of the face (role_a) and that of the rest, to be
+// mixed as a_sig fA + (1 - a_sig) fB; both lanes get the whole flux where
+// neither cell is a mixture of the two (returns false).  With A the lane's own
+// material and B the other, and a pure cell standing for both its parts, every
+// branch of the reference is one of hllc(L_A, R_A), classic(L_B, L_A, R_A) and
+// inverse(L_A, R_A, R_B); inverse (CrpFlux::inverse, crp_flux.cpp:493-512) is the
+// classic problem mirrored in x (PState::inverse flips u, Flux::inverse negates
+// all but m_x, models.cpp:219-221, 506-515).  So the lanes differ in selected
+// inputs and not in their paths: with the reference's branches inlined, one
+// wavefront walked through up to six copies of the classic problem.
+template <int NM>
+__device__ __forceinline__ bool calc_crp_part(const MZ<NM>& zL, const MZ<NM>& zR, double hL, double hR, int iA,
+                                              double a_sig, double dt, const Mix& mx, bool role_a, double* F,
+                                              bool& err) {
+    const double aL = alpha_of<NM>(zL, iA), aR = alpha_of<NM>(zR, iA);
+    const bool pureL = aL == 0.0 || aL == 1.0, pureR = aR == 0.0 || aR == 1.0;
+    MZ<NM> LA = zL, LB = zL, RA = zR, RB = zR;
+    if (!pureL) m_split<NM>(zL, mx, iA, LA, LB);
+    if (!pureR) m_split<NM>(zR, mx, iA, RA, RB);
+    // the lane's own part of either side, and the other part
+    const MZ<NM> Lo = select_mz<NM>(role_a, LA, LB), Lx = select_mz<NM>(role_a, LB, LA);
+    const MZ<NM> Ro = select_mz<NM>(role_a, RA, RB), Rx = select_mz<NM>(role_a, RB, RA);
+    bool plain, inverse;
+    if (aL == 0.0 || aL == 1.0) {
+        plain = (aL == 0.0) == role_a;
+        inverse = true;
+    } else if (pureR) {
+        plain = (aR == 0.0) == role_a;
+        inverse = false;
+    } else {
+        plain = false;
+        inverse = (aL < aR) != role_a;
+    }
+    if ((pureL && pureR) || plain) {
+        hllc_mm<NM>(Lo, Ro, F, err);
+    } else {
+        const double delta_L = (aL < a_sig ? aL / a_sig : (1.0 - aL) / (1.0 - a_sig)) * hL;
+        const double delta_R = (aR < a_sig ? aR / a_sig : (1.0 - aR) / (1.0 - a_sig)) * hR;
+        MZ<NM> p = select_mz<NM>(inverse, Rx, Lx), q = select_mz<NM>(inverse, Ro, Lo),
+               r = select_mz<NM>(inverse, Lo, Ro);
+        p.u = inverse ? -p.u : p.u;
+        q.u = inverse ? -q.u : q.u;
+        r.u = inverse ? -r.u : r.u;
+        crp_classic<NM>(p, q, r, mx, inverse ? delta_R : delta_L, dt, F, err);
+#pragma unroll
+        for (int k = 0; k < 4 + NM; ++k)
+            if (k != 1) F[k] = inverse ? -F[k] : F[k];
+    }
+    return !(pureL && pureR);
 }
 
 // average_flux (geom/sections.cpp:125-148) and between (math/funcs.h:47-50).
