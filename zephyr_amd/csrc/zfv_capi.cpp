@@ -223,7 +223,7 @@ struct zfv_ctx {
         int limiter = 3;              // MC (mm_fluid.cpp:20)
         int acc = 1;                  // m_acc (mm_fluid.h:157)
         DBuf<int> crp_list, crp_cells;
-        DBuf<unsigned int> crp_count;   // [0] listed faces, [1] listed cells
+        DBuf<unsigned int> crp_count;   // [0] listed faces, [1] listed cells, [2] the last sweep's faces
         DBuf<unsigned long long> dtmin;
         // The composite fluxes on a second stream (same priority), beside
         // the update of the cells without a composite face: `side` and the
@@ -2636,7 +2636,10 @@ int zfv_mm_step(zfv_ctx* ctx, int n_steps) {
         if (S.inter.n != 3 * nm * cap) ZFV_HIP(S.inter.alloc(3 * nm * cap));
         if (S.cf.n != 8 * (4 + nm) * cap) ZFV_HIP(S.cf.alloc(8 * (4 + nm) * cap));
         if (S.crp_list.n != 8 * cap) ZFV_HIP(S.crp_list.alloc(8 * cap));
-        if (S.crp_count.n != 2) ZFV_HIP(S.crp_count.alloc(2));
+        if (S.crp_count.n != 4) {
+            ZFV_HIP(S.crp_count.alloc(4));
+            ZFV_HIP(launch_fill_u64((unsigned long long*)S.crp_count.p, 2, 0ULL, ctx->stream));
+        }
         if (S.overlap) {
             if (S.overlap == 2 && S.crp_cells.n != cap) ZFV_HIP(S.crp_cells.alloc(cap));
             if (!S.side) ZFV_HIP(hipStreamCreateWithFlags(&S.side, hipStreamNonBlocking));
@@ -2684,7 +2687,9 @@ int zfv_mm_step(zfv_ctx* ctx, int n_steps) {
                 ZFV_HIP(hipEventRecord(S.ev_in, s1));   // `in` is complete
                 ZFV_HIP(hipStreamWaitEvent(s2, S.ev_in, 0));
             }
-            if (plic) {   // interface_recovery (mm_fluid.cpp:143-146, 160-163)
+            // interface_recovery (mm_fluid.cpp:143-146, 160-163): with the marking, or (modes 1 and 2) beside it
+            const MmInterface inter{ctx->vx.p, ctx->vy.p, ir, ir + nm * cap, ir + 2 * nm * cap};
+            if (plic && mode) {
                 ZFV_HIP(timed_on(ctx, s2, "mm_interface", [&] {
                     return mm_interface(M, in, S.mix, ctx->vx.p, ctx->vy.p, ir, ir + nm * cap, ir + 2 * nm * cap, s2);
                 }));
@@ -2701,7 +2706,8 @@ int zfv_mm_step(zfv_ctx* ctx, int n_steps) {
             if (S.crp) {   // the composite fluxes of the sweep's faces
                 ZFV_HIP(timed(ctx, "mm_crp_mark", [&] {
                     return mm_crp_mark(M, in, half, S.mix, acc, o, S.gx.p, S.gy.p, S.crp_list.p,
-                                       mode == 2 ? S.crp_cells.p : nullptr, S.crp_count.p, s1);
+                                       mode == 2 ? S.crp_cells.p : nullptr, S.crp_count.p,
+                                       plic && !mode ? &inter : nullptr, s1);
                 }));
                 // the composite fluxes run where the interface ran (s2),
                 // after the marking; mode 1 joins before them
@@ -2735,6 +2741,7 @@ int zfv_mm_step(zfv_ctx* ctx, int n_steps) {
             if (mode == 2) {
                 ZFV_HIP(hipStreamWaitEvent(s1, S.ev_crp, 0));
                 ZFV_HIP(update(2));
+                ZFV_HIP(mm_take_count(S.crp_count.p, s1));
             }
             S.cur = 1 - S.cur;   // MmFluid::swap, after every integrate
         }
@@ -2755,7 +2762,7 @@ int zfv_mm_crp_faces(zfv_ctx* ctx, int64_t* n) {
     if (!n) return fail(ZFV_ERR_ARG, "null output");
     unsigned int k = 0;
     if (ctx->mm.crp && ctx->mm.crp_count.p) {
-        ZFV_HIP(hipMemcpyAsync(&k, ctx->mm.crp_count.p, sizeof(k), hipMemcpyDeviceToHost, ctx->stream));
+        ZFV_HIP(hipMemcpyAsync(&k, ctx->mm.crp_count.p + 2, sizeof(k), hipMemcpyDeviceToHost, ctx->stream));
         ZFV_HIP(hipStreamSynchronize(ctx->stream));
     }
     *n = k;

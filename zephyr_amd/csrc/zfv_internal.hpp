@@ -295,19 +295,28 @@ hipError_t mm_prepare(const DevMesh& M, const MmLayer& L, const mm::Mix& mx, uns
 // or null without composite Riemann problems.  pass 0: every cell; pass 1:
 // the cells without a composite face (CF is not read: mm_crp may still be
 // writing it on another stream); pass 2: the cells listed by mm_crp_mark
-// (cells, count[1]), which pass 1 left.
+// (cells, count[1]), which pass 1 left.  Pass 0 takes the counters (with CF);
+// after pass 2 mm_take_count does.
 hipError_t mm_flux1(const DevMesh& M, const MmLayer& in, const MmLayer& out, const mm::Mix& mx,
                     const StepCtl& ctl, const MmOpts& o, const double* CF, int pass, const int* cells,
-                    const unsigned int* count, hipStream_t s);
+                    unsigned int* count, hipStream_t s);
+hipError_t mm_take_count(unsigned int* count, hipStream_t s);
 // The faces that take composite Riemann fluxes: list (8 * stride ints of
 // work space) and their number (count[0]), with `cells` (stride ints, or
 // null) the cells that have such a face and their number (count[1]); then
 // the fluxes into CF, over `groups` one-wavefront workgroups.  acc 1 reads
 // the cells of `in`; acc 2 the face states extrapolated from `half` with
-// the gradients gx / gy ([6 + 2 n_mat][stride], k_mm_grad).
+// the gradients gx / gy ([6 + 2 n_mat][stride], k_mm_grad).  count[0] and
+// count[1] are clear before the marking and cleared again when taken; count[2]
+// is the last taken count[0].  With `inter` the marking also does mm_interface
+// of `in`.
+struct MmInterface {
+    const double *vx, *vy;
+    double *nx, *ny, *p;
+};
 hipError_t mm_crp_mark(const DevMesh& M, const MmLayer& in, const MmLayer& half, const mm::Mix& mx, int acc,
                        const MmOpts& o, const double* gx, const double* gy, int* list, int* cells,
-                       unsigned int* count, hipStream_t s);
+                       unsigned int* count, const MmInterface* inter, hipStream_t s);
 hipError_t mm_crp(const DevMesh& M, const MmLayer& in, const MmLayer& half, const mm::Mix& mx, int acc,
                   const MmOpts& o, const double* gx, const double* gy, const StepCtl& ctl, const double* nx,
                   const double* ny, const int* list, const unsigned int* count, double* CF, int groups,
@@ -317,7 +326,7 @@ hipError_t mm_stage1(const DevMesh& M, const MmLayer& in, const MmLayer& half, c
                      const MmOpts& o, const double* gx, const double* gy, hipStream_t s);
 hipError_t mm_flux2(const DevMesh& M, const MmLayer& in, const MmLayer& half, const MmLayer& out, const mm::Mix& mx,
                     const StepCtl& ctl, const MmOpts& o, const double* gx, const double* gy, const double* CF,
-                    int pass, const int* cells, const unsigned int* count, hipStream_t s);
+                    int pass, const int* cells, unsigned int* count, hipStream_t s);
 hipError_t mm_interface(const DevMesh& M, const MmLayer& L, const mm::Mix& mx, const double* vx, const double* vy,
                         double* nx, double* ny, double* p, hipStream_t s);
 // Adaptation of the multi-material state: the limited gradient (rows rho,

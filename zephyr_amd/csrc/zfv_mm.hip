@@ -247,33 +247,188 @@ __device__ __forceinline__ bool crp_face(const double* CF, const MZ<NM>& zm, con
     return CF != nullptr && !(frac_index<NM>(zm.b) >= 0 && frac_index<NM>(zp.b) >= 0);
 }
 
+// A cell's neighbours across slots s0 to s0 + 3 (itself where there is none),
+// all loaded before any is used: one round trip in place of one a slot.
+__device__ __forceinline__ void mm_neighbours(const DevMesh& M, int c, int code, int s0, int* nb) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int t = (code >> (4 * (s0 + k))) & 7;
+        nb[k] = t != SC_UNDEF && t < SC_WALL ? M.adj[(s0 + k) * M.stride + c] : c;
+    }
+}
+
+// MmFluid::interface_recovery (mm_fluid.cpp:484-519): per mixed cell and
+// present material, n = -sum_faces face_fraction(alpha_c, alpha_n) S n_f,
+// normalised, and the section position p = quad_find_section(alpha_c, n,
+// hx, hy) (geom/sections.cpp:25-37); zero for pure cells.
+template <int NM>
+__device__ __forceinline__ void mm_interface_cell(const DevMesh& M, const MmLayer& L, const double* __restrict__ vx,
+                                                  const double* __restrict__ vy, double* __restrict__ onx,
+                                                  double* __restrict__ ony, double* __restrict__ op, int c, int code) {
+    const int st = M.stride;
+    double b[NM], nsx[NM], nsy[NM], ps[NM];
+#pragma unroll
+    for (int i = 0; i < NM; ++i) {
+        b[i] = L.b[i * st + c];
+        nsx[i] = 0.0;
+        nsy[i] = 0.0;
+        ps[i] = 0.0;
+    }
+    if (!frac_pure<NM>(b)) {
+        const double r = L.r[c];
+        double a_c[NM];
+#pragma unroll
+        for (int i = 0; i < NM; ++i) a_c[i] = b[i] > 0.0 ? b[i] * r / L.rh[i * st + c] : 0.0;   // volume_fractions
+        double wx[4], wy[4];   // the middles of the sides
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            wx[k] = vx[(k == 0 ? 5 : (k == 1 ? 3 : (k == 2 ? 7 : 1))) * st + c];
+            wy[k] = vy[(k == 0 ? 5 : (k == 1 ? 3 : (k == 2 ? 7 : 1))) * st + c];
+        }
+#pragma unroll 1
+        for (int s0 = 0; s0 < 8; s0 += 4) {
+            if (((code >> (4 * s0)) & 0x7777) == SC_UNDEF * 0x1111) continue;
+            // the four slots' loads, then their sums in slot order; neib() is the cell itself at a boundary
+            int nb[4];
+            double Sx[4], Sy[4], rn[4], rhn[4][NM], bn[4][NM];
+            mm_neighbours(M, c, code, s0, nb);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int so = (s0 + k) * st + c;
+                const double a = M.area[so];
+                Sx[k] = a * M.nx[so];
+                Sy[k] = a * M.ny[so];
+                rn[k] = L.r[nb[k]];
+#pragma unroll
+                for (int i = 0; i < NM; ++i) {
+                    rhn[k][i] = L.rh[i * st + nb[k]];
+                    bn[k][i] = L.b[i * st + nb[k]];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (((code >> (4 * (s0 + k))) & 7) == SC_UNDEF) continue;
+#pragma unroll
+                for (int i = 0; i < NM; ++i) {
+                    if (!(a_c[i] > 0.0)) continue;
+                    double a_n = 0.0;   // PState::alpha (models.cpp:224-227)
+                    if (!isnan(rhn[k][i])) {
+                        const double x = bn[k][i] * rn[k] / rhn[k][i];
+                        const double lo = (1.0 < x) ? 1.0 : x;
+                        a_n = (0.0 < lo) ? lo : 0.0;
+                    }
+                    const double ff = face_fraction(a_c[i], a_n);
+                    nsx[i] = nsx[i] - ff * Sx[k];
+                    nsy[i] = nsy[i] - ff * Sy[k];
+                }
+            }
+        }
+        const double hx = sqrt((wx[0] - wx[1]) * (wx[0] - wx[1]) + (wy[0] - wy[1]) * (wy[0] - wy[1]));
+        const double hy = sqrt((wx[2] - wx[3]) * (wx[2] - wx[3]) + (wy[2] - wy[3]) * (wy[2] - wy[3]));
+#pragma unroll
+        for (int i = 0; i < NM; ++i) {
+            if (!(a_c[i] > 0.0)) continue;
+            const double zz = nsx[i] * nsx[i] + nsy[i] * nsy[i];
+            if (zz > 0.0) {
+                const double q = sqrt(zz);
+                nsx[i] = nsx[i] / q;
+                nsy[i] = nsy[i] / q;
+            }
+            ps[i] = quad_find_section(a_c[i], nsx[i], nsy[i], hx, hy);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NM; ++i) {
+        onx[i * st + c] = nsx[i];
+        ony[i * st + c] = nsy[i];
+        op[i * st + c] = ps[i];
+    }
+}
+
+template <int NM>
+__global__ void __launch_bounds__(kBlock) k_mm_interface(DevMesh M, MmLayer L, const double* __restrict__ vx,
+                                                         const double* __restrict__ vy, double* __restrict__ onx,
+                                                         double* __restrict__ ony, double* __restrict__ op) {
+    const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (c < M.n) mm_interface_cell<NM>(M, L, vx, vy, onx, ony, op, c, M.code[c]);
+}
+
 // Faces that need a composite Riemann flux (CrpMode::PLIC): a mixed face
 // state on either side (MmFluid::calc_flux, mm_fluid.cpp:347-371; a
 // boundary face's other side is the boundary value of the cell's own).  acc
 // 1: the cells' states; acc 2: the extrapolated, normalised half states.
 // Appends slot-major pairs s * stride + c to `list` (counter count[0]) and,
 // when `cells` is given, each cell with such a face to `cells` (counter
-// count[1]); the counters start at zero.
-template <int NM, int ACC>
+// count[1]); the counters start at zero, and a wavefront adds to each once.
+// INTER: also the interface reconstruction of `in` (mm_interface_cell), whose
+// mixed cells are among the marked ones; what bounds either alone is its chain
+// of loads (384^2 cells: a launch for each and one for the counters 18 + 20 us,
+// 18 together).
+template <int NM, int ACC, bool INTER>
 __global__ void __launch_bounds__(kBlock) k_mm_crp_mark(DevMesh M, MmLayer in, MmLayer half,
                                                         const double* __restrict__ gx, const double* __restrict__ gy,
                                                         int dir, int* __restrict__ list, int* __restrict__ cells,
-                                                        unsigned int* count) {
+                                                        unsigned int* count, const double* __restrict__ vx,
+                                                        const double* __restrict__ vy, double* __restrict__ onx,
+                                                        double* __restrict__ ony, double* __restrict__ op) {
     const Tile tl = tile_of(M, (int)blockDim.x);
     const int c = tl.c0 + (int)threadIdx.x;
-    if (c >= tl.end) return;
     const int st = M.stride;
-    const int code = M.code[c];
-    bool any = false;
-    for (int s = 0; s < 8; ++s) {
-        const int t = (code >> (4 * s)) & 7;
-        if (t == SC_UNDEF || !mm_swept(M, s * st + c, dir)) continue;
-        if (mm_crp_slot<NM, ACC>(M, in, half, gx, gy, c, s * st + c, t)) {
-            list[atomicAdd(count, 1u)] = s * st + c;
-            any = true;
+    unsigned marks = 0u;   // bit s: slot s is listed
+    if (c < tl.end) {
+        const int code = M.code[c];
+        if (ACC == 1) {
+            double b[NM];
+#pragma unroll
+            for (int i = 0; i < NM; ++i) b[i] = in.b[i * st + c];
+            const bool own = frac_index<NM>(b) < 0;
+#pragma unroll
+            for (int s0 = 0; s0 < 8; s0 += 4) {
+                if (((code >> (4 * s0)) & 0x7777) == SC_UNDEF * 0x1111) continue;
+                int nb[4];
+                double bn[4][NM];
+                mm_neighbours(M, c, code, s0, nb);
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int i = 0; i < NM; ++i) bn[k][i] = in.b[i * st + nb[k]];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int t = (code >> (4 * (s0 + k))) & 7;
+                    const bool mixed = own || (t <= SC_PERIODIC && frac_index<NM>(bn[k]) < 0);
+                    if (t != SC_UNDEF && mixed && mm_swept(M, (s0 + k) * st + c, dir)) marks |= 1u << (s0 + k);
+                }
+            }
+        } else {
+#pragma unroll 1
+            for (int s = 0; s < 8; ++s) {
+                const int t = (code >> (4 * s)) & 7;
+                if (t == SC_UNDEF || !mm_swept(M, s * st + c, dir)) continue;
+                if (mm_crp_slot<NM, ACC>(M, in, half, gx, gy, c, s * st + c, t)) marks |= 1u << s;
+            }
         }
+        if (INTER) mm_interface_cell<NM>(M, in, vx, vy, onx, ony, op, c, code);
     }
-    if (any && cells) cells[atomicAdd(count + 1, 1u)] = c;
+    if (__ballot(marks != 0u) == 0ULL) return;
+    const unsigned long long below = (1ULL << (threadIdx.x & 63)) - 1ULL;
+    int total = 0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) total += __popcll(__ballot((marks >> s) & 1u));
+    const unsigned long long any = __ballot(marks != 0u);
+    int at = 0, cell_at = 0;
+    if ((threadIdx.x & 63) == 0) {
+        at = (int)atomicAdd(count, (unsigned)total);
+        if (cells) cell_at = (int)atomicAdd(count + 1, (unsigned)__popcll(any));
+    }
+    at = __builtin_amdgcn_readfirstlane(at);
+    cell_at = __builtin_amdgcn_readfirstlane(cell_at);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const unsigned long long m = __ballot((marks >> s) & 1u);
+        if ((marks >> s) & 1u) list[at + __popcll(m & below)] = s * st + c;
+        at += __popcll(m);
+    }
+    if (cells && marks != 0u) cells[cell_at + __popcll(any & below)] = c;
 }
 
 // The composite Riemann flux of each listed face, two lanes a face: the
@@ -423,15 +578,29 @@ __device__ __forceinline__ double mm_flux1_cell(const DevMesh& M, const MmLayer&
     return mm_dt_cand<NM>(M, c, zn);
 }
 
+// The sweep's counters, once nothing reads them any more: count[2] keeps the
+// number of listed faces, the others are left clear for the next marking.
+__device__ __forceinline__ void take_count(unsigned int* count) {
+    count[2] = count[0];
+    count[0] = 0u;
+    count[1] = 0u;
+}
+__global__ void __launch_bounds__(64) k_mm_take_count(unsigned int* count) {
+    if (threadIdx.x == 0) take_count(count);
+}
+
 // Every cell (defer = false), or every cell without a composite face
-// (defer = true, while k_mm_crp fills CF on another stream).
+// (defer = true, while k_mm_crp fills CF on another stream).  `done`: the
+// marking's counters, taken here where every cell is updated.
 template <int NM, int PLAIN>
 __global__ void __launch_bounds__(kBlock) k_mm_flux1(DevMesh M, MmLayer in, MmLayer out, Mix mx, StepCtl ctl,
-                                                     MmOpts opt, const double* __restrict__ CF, int defer) {
+                                                     MmOpts opt, const double* __restrict__ CF, int defer,
+                                                     unsigned int* done) {
     const Tile tl = tile_of(M, (int)blockDim.x);
     const int c = tl.c0 + (int)threadIdx.x;
     const double step = step_dt(ctl, tl.pid);
     step_prologue(ctl, tl, step);
+    if (done && blockIdx.x == 0 && threadIdx.x == 0) take_count(done);
     const double dt = opt.dt_scale * step;
     double cand = INFINITY;
     if (c < tl.end) cand = mm_flux1_cell<NM, PLAIN>(M, in, out, mx, ctl, opt, CF, c, dt, defer != 0);
@@ -566,11 +735,12 @@ template <int NM, int PLAIN>
 __global__ void __launch_bounds__(kBlock) k_mm_flux2(DevMesh M, MmLayer in, MmLayer half, MmLayer out, Mix mx,
                                                      StepCtl ctl, MmOpts opt, const double* __restrict__ gx,
                                                      const double* __restrict__ gy, const double* __restrict__ CF,
-                                                     int defer) {
+                                                     int defer, unsigned int* done) {
     const Tile tl = tile_of(M, (int)blockDim.x);
     const int c = tl.c0 + (int)threadIdx.x;
     const double step = step_dt(ctl, tl.pid);
     step_prologue(ctl, tl, step);
+    if (done && blockIdx.x == 0 && threadIdx.x == 0) take_count(done);
     const double dt = opt.dt_scale * step;
     double cand = INFINITY;
     if (c < tl.end) cand = mm_flux2_cell<NM, PLAIN>(M, in, half, out, mx, ctl, opt, gx, gy, CF, c, dt, defer != 0);
@@ -592,78 +762,6 @@ __global__ void __launch_bounds__(kBlock) k_mm_flux2_list(DevMesh M, MmLayer in,
         cand = v < cand ? v : cand;
     }
     block_min_atomic(&ctl.dtmin[ctl.wr], cand);
-}
-
-// MmFluid::interface_recovery (mm_fluid.cpp:484-519): per mixed cell and
-// present material, n = -sum_faces face_fraction(alpha_c, alpha_n) S n_f,
-// normalised, and the section position p = quad_find_section(alpha_c, n,
-// hx, hy) (geom/sections.cpp:25-37); zero for pure cells.
-template <int NM>
-__global__ void __launch_bounds__(kBlock) k_mm_interface(DevMesh M, MmLayer L, const double* __restrict__ vx,
-                                                         const double* __restrict__ vy, double* __restrict__ onx,
-                                                         double* __restrict__ ony, double* __restrict__ op) {
-    const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (c >= M.n) return;
-    const int st = M.stride;
-    const MZ<NM> z = load_mz<NM>(L, c, st);
-    double nsx[NM], nsy[NM], ps[NM];
-#pragma unroll
-    for (int i = 0; i < NM; ++i) {
-        nsx[i] = 0.0;
-        nsy[i] = 0.0;
-        ps[i] = 0.0;
-    }
-    if (!frac_pure<NM>(z.b)) {
-        double a_c[NM];
-#pragma unroll
-        for (int i = 0; i < NM; ++i) a_c[i] = z.b[i] > 0.0 ? z.b[i] * z.r / z.rh[i] : 0.0;   // volume_fractions
-        const int code = M.code[c];
-#pragma unroll 1
-        for (int s = 0; s < 8; ++s) {
-            const int t = (code >> (4 * s)) & 7;
-            if (t == SC_UNDEF) continue;
-            const int so = s * st + c;
-            const double a = M.area[so];
-            const double Sx = a * M.nx[so], Sy = a * M.ny[so];
-            const int nb = t >= SC_WALL ? c : M.adj[so];   // neib() is the cell itself at a boundary
-            const double rn = L.r[nb];
-#pragma unroll
-            for (int i = 0; i < NM; ++i) {
-                if (!(a_c[i] > 0.0)) continue;
-                const double rhn = L.rh[i * st + nb];
-                double a_n = 0.0;   // PState::alpha (models.cpp:224-227)
-                if (!isnan(rhn)) {
-                    const double x = L.b[i * st + nb] * rn / rhn;
-                    const double lo = (1.0 < x) ? 1.0 : x;
-                    a_n = (0.0 < lo) ? lo : 0.0;
-                }
-                const double ff = face_fraction(a_c[i], a_n);
-                nsx[i] = nsx[i] - ff * Sx;
-                nsy[i] = nsy[i] - ff * Sy;
-            }
-        }
-        const double hx = sqrt((vx[5 * st + c] - vx[3 * st + c]) * (vx[5 * st + c] - vx[3 * st + c]) +
-                               (vy[5 * st + c] - vy[3 * st + c]) * (vy[5 * st + c] - vy[3 * st + c]));
-        const double hy = sqrt((vx[7 * st + c] - vx[1 * st + c]) * (vx[7 * st + c] - vx[1 * st + c]) +
-                               (vy[7 * st + c] - vy[1 * st + c]) * (vy[7 * st + c] - vy[1 * st + c]));
-#pragma unroll
-        for (int i = 0; i < NM; ++i) {
-            if (!(a_c[i] > 0.0)) continue;
-            const double zz = nsx[i] * nsx[i] + nsy[i] * nsy[i];
-            if (zz > 0.0) {
-                const double r = sqrt(zz);
-                nsx[i] = nsx[i] / r;
-                nsy[i] = nsy[i] / r;
-            }
-            ps[i] = quad_find_section(a_c[i], nsx[i], nsy[i], hx, hy);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < NM; ++i) {
-        onx[i * st + c] = nsx[i];
-        ony[i * st + c] = nsy[i];
-        op[i * st + c] = ps[i];
-    }
 }
 
 // ---- adaptation: MmFluid::compute_grad, set_flags, distributor --------------
@@ -1039,7 +1137,7 @@ hipError_t mm_prepare(const DevMesh& M, const MmLayer& L, const Mix& mx, unsigne
 }
 
 hipError_t mm_flux1(const DevMesh& M, const MmLayer& in, const MmLayer& out, const Mix& mx, const StepCtl& ctl,
-                    const MmOpts& o, const double* CF, int pass, const int* cells, const unsigned int* count,
+                    const MmOpts& o, const double* CF, int pass, const int* cells, unsigned int* count,
                     hipStream_t s) {
     const int plain = o.flux == kFluxHllc ? 1 : 2;
     if (pass == 2) {
@@ -1047,22 +1145,37 @@ hipError_t mm_flux1(const DevMesh& M, const MmLayer& in, const MmLayer& out, con
                             o, CF, cells, count);
     } else {
         ZFV_MM_DISPATCH_ACC(mx.n, plain, k_mm_flux1, mm_grid(M.n), dim3(kBlock), 0, s, M, in, out, mx, ctl, o, CF,
-                            pass);
+                            pass, pass == 0 && CF ? count : nullptr);
     }
     return hipGetLastError();
 }
 
-__global__ void __launch_bounds__(64) k_zero_u32(unsigned int* p) {
-    if (threadIdx.x < 2) p[threadIdx.x] = 0u;
-}
-
 hipError_t mm_crp_mark(const DevMesh& M, const MmLayer& in, const MmLayer& half, const Mix& mx, int acc,
                        const MmOpts& o, const double* gx, const double* gy, int* list, int* cells,
-                       unsigned int* count, hipStream_t s) {
-    // the counters are cleared by a kernel, not a memset node, so the step can be captured
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, count);
-    ZFV_MM_DISPATCH_ACC(mx.n, acc, k_mm_crp_mark, mm_grid(M.n), dim3(kBlock), 0, s, M, in, half, gx, gy, o.dir,
-                        list, cells, count);
+                       unsigned int* count, const MmInterface* inter, hipStream_t s) {
+#define ZFV_MM_MARK(NMC, A)                                                                                      \
+    if (inter)                                                                                                   \
+        hipLaunchKernelGGL((k_mm_crp_mark<NMC, A, true>), mm_grid(M.n), dim3(kBlock), 0, s, M, in, half, gx, gy, o.dir, \
+                           list, cells, count, inter->vx, inter->vy, inter->nx, inter->ny, inter->p);            \
+    else                                                                                                         \
+        hipLaunchKernelGGL((k_mm_crp_mark<NMC, A, false>), mm_grid(M.n), dim3(kBlock), 0, s, M, in, half, gx, gy,  \
+                           o.dir, list, cells, count, nullptr, nullptr, nullptr, nullptr, nullptr)
+    switch (mx.n * 2 + acc - 1) {
+        case 2: ZFV_MM_MARK(1, 1); break;
+        case 3: ZFV_MM_MARK(1, 2); break;
+        case 4: ZFV_MM_MARK(2, 1); break;
+        case 5: ZFV_MM_MARK(2, 2); break;
+        case 6: ZFV_MM_MARK(3, 1); break;
+        case 7: ZFV_MM_MARK(3, 2); break;
+        case 8: ZFV_MM_MARK(4, 1); break;
+        default: ZFV_MM_MARK(4, 2); break;
+    }
+#undef ZFV_MM_MARK
+    return hipGetLastError();
+}
+
+hipError_t mm_take_count(unsigned int* count, hipStream_t s) {
+    hipLaunchKernelGGL(k_mm_take_count, dim3(1), dim3(64), 0, s, count);
     return hipGetLastError();
 }
 
@@ -1084,14 +1197,14 @@ hipError_t mm_stage1(const DevMesh& M, const MmLayer& in, const MmLayer& half, c
 
 hipError_t mm_flux2(const DevMesh& M, const MmLayer& in, const MmLayer& half, const MmLayer& out, const Mix& mx,
                     const StepCtl& ctl, const MmOpts& o, const double* gx, const double* gy, const double* CF,
-                    int pass, const int* cells, const unsigned int* count, hipStream_t s) {
+                    int pass, const int* cells, unsigned int* count, hipStream_t s) {
     const int plain = o.flux == kFluxHllc ? 1 : 2;
     if (pass == 2) {
         ZFV_MM_DISPATCH_ACC(mx.n, plain, k_mm_flux2_list, dim3(kListGroups), dim3(kBlock), 0, s, M, in, half, out,
                             mx, ctl, o, gx, gy, CF, cells, count);
     } else {
         ZFV_MM_DISPATCH_ACC(mx.n, plain, k_mm_flux2, mm_grid(M.n), dim3(kBlock), 0, s, M, in, half, out, mx, ctl, o,
-                            gx, gy, CF, pass);
+                            gx, gy, CF, pass, pass == 0 && CF ? count : nullptr);
     }
     return hipGetLastError();
 }
