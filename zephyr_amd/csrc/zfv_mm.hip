@@ -807,11 +807,12 @@ __device__ __forceinline__ const double* mg_row(const MmLayer& L, int st, int k)
 // component as k_grad_pred does for SmFluid (the 2 x 2 block of the LSM
 // system).  The first `rows` of the 6 + 2 NM components (all of them for a
 // second-order step, the 4 + NM the split distributor reads for
-// set_flags) go in chunks of KC through the two passes (the unlimited and
-// the limited right-hand side), so a thread holds KC components' sums
-// rather than all of them; the LSM matrix is built in the first chunk's
-// first pass.  Each component's sums run over the slots in the same order
-// as unchunked, so the result does not depend on KC.  gx, gy:
+// set_flags) go in chunks of KC through the two passes (the unlimited and the
+// limited right-hand side), so a thread holds KC components' sums rather than
+// all of them; the LSM matrix is built in its first chunk's first pass.  On small
+// meshes, where a thread's time is its chain of loads slot by slot, a row of the
+// grid takes each chunk (kGradSplit).  Each component's sums run over the slots
+// in the same order, so the result does not depend on KC or the rows.  gx, gy:
 // [6 + 2 NM][stride].
 template <int NM, int KC>
 __global__ void __launch_bounds__(kBlock) k_mm_grad(DevMesh M, MmLayer L, int crp, int limiter, int rows,
@@ -835,18 +836,20 @@ __global__ void __launch_bounds__(kBlock) k_mm_grad(DevMesh M, MmLayer L, int cr
             if (frac_index<NM>(b) < 0) zero = true;
         }
     }
+    const int kb = (int)blockIdx.y * KC, ks = (int)gridDim.y * KC;
     if (zero) {
-        for (int k = 0; k < rows; ++k) {
-            gx[k * st + c] = 0.0;
-            gy[k * st + c] = 0.0;
-        }
+        for (int k0 = kb; k0 < rows; k0 += ks)
+            for (int k = k0; k < rows && k < k0 + KC; ++k) {
+                gx[k * st + c] = 0.0;
+                gy[k * st + c] = 0.0;
+            }
         return;
     }
     const double ccx = M.cx[c], ccy = M.cy[c];
     double A00 = 0.0, A01 = 0.0, A10 = 0.0, A11 = 0.0;
     double B00 = 0.0, B01 = 0.0, B10 = 0.0, B11 = 0.0;
 #pragma unroll 1
-    for (int k0 = 0; k0 < rows; k0 += KC) {
+    for (int k0 = kb; k0 < rows; k0 += ks) {
         double zc[KC], Gx[KC], Gy[KC];
 #pragma unroll
         for (int j = 0; j < KC; ++j) {
@@ -894,7 +897,7 @@ __global__ void __launch_bounds__(kBlock) k_mm_grad(DevMesh M, MmLayer L, int cr
                 }
                 const bool xp = fr.gen || fr.side < 2, yp = fr.gen || fr.side >= 2;
                 const double w = M.w[so];
-                if (k0 == 0 && pass == 0) {   // the LSM matrix
+                if (k0 == kb && pass == 0) {   // the LSM matrix
                     if (xp) {
                         const double wd = w * dnx;
                         A00 = A00 + wd * drx;
@@ -918,7 +921,7 @@ __global__ void __launch_bounds__(kBlock) k_mm_grad(DevMesh M, MmLayer L, int cr
                     if (yp) Fy[j] = Fy[j] + (w * term) * dny;
                 }
             }
-            if (k0 == 0 && pass == 0) {   // its inverse
+            if (k0 == kb && pass == 0) {   // its inverse
                 if (fabs(A11) < 1e-8) A11 = 1.0;
                 const double det = A11 * A00 + (-A01) * A10;
                 const double invdet = 1.0 / det;
@@ -1108,6 +1111,11 @@ __global__ void __launch_bounds__(kBlock) k_mm_cache(DevMesh M, MmLayer L, Mix m
 static inline dim3 mm_grid(int n) { return dim3((n + kBlock - 1) / kBlock); }
 // workgroups of the deferred-cell passes (a few thousand cells at most, grid-stride)
 constexpr int kListGroups = 64;
+// k_mm_grad takes its chunks beside each other up to this many cells.  Second-order
+// steps of two materials, beside / in turn: 6400 cells 17 / 35 us, 73745 26 / 43,
+// 250000 72 / 66, 1000000 249 / 229 (the chip is full, and the cells' own loads are
+// made once a chunk).
+constexpr int kGradSplit = 131072;
 
 #define ZFV_MM_DISPATCH(NMAT, KERNEL, ...)                                                              \
     switch (NMAT) {                                                                                     \
@@ -1221,8 +1229,12 @@ hipError_t mm_grad(const DevMesh& M, const MmLayer& L, const Mix& mx, int crp, i
     // the rows of set_flags (4 + NM) in one chunk; all 6 + 2 NM of a
     // second-order step in chunks of 4, which keeps more wavefronts resident
     const bool split = rows <= 4 + mx.n;
+    auto grid = [&](int nm) {
+        const int kc = split ? 4 + nm : 4;
+        return dim3(mm_grid(M.n).x, M.n <= kGradSplit ? (unsigned)((rows + kc - 1) / kc) : 1u);
+    };
 #define ZFV_MM_GRAD(NMC)                                                                                     \
-    hipLaunchKernelGGL((split ? k_mm_grad<NMC, 4 + NMC> : k_mm_grad<NMC, 4>), mm_grid(M.n), dim3(kBlock), 0, s, \
+    hipLaunchKernelGGL((split ? k_mm_grad<NMC, 4 + NMC> : k_mm_grad<NMC, 4>), grid(NMC), dim3(kBlock), 0, s, \
                        M, L, crp, limiter, rows, gx, gy)
     switch (mx.n) {
         case 1: ZFV_MM_GRAD(1); break;
