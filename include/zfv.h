@@ -432,17 +432,19 @@ int zfv_restore(zfv_ctx* ctx, const char* root);
  * (one face each), 2 = one thread per cell with the main slots' loads
  * issued together (more registers per thread; for meshes that do not fill
  * the GPU), block = workgroup size 128, 256 or 512 (0 keeps the current
- * one).  Layout 3 (stage 1 only) runs the whole MUSCL + HLLC step in one
- * tiled kernel with the half states and gradients in LDS, on meshes built
- * by zfv_mesh_rectangle / zfv_batch_rectangles (before any adaptation;
- * ZFV_ERR_UNSUPPORTED otherwise); its block is the tile shape, 512, 768 or
- * 1024 threads (6, 10 or 14 rows of 62 cells); it is the default there, and
- * schemes it does not cover run the stage kernels.  All choices give
- * bit-identical results. */
+ * one).  Layout 3 (stage 1 only) runs the whole MUSCL step with the HLLC, HLL
+ * or Rusanov flux in one tiled kernel with the half states and gradients in
+ * LDS, on meshes built by zfv_mesh_rectangle / zfv_batch_rectangles (before any
+ * adaptation; ZFV_ERR_UNSUPPORTED otherwise); its block is the tile shape, 512,
+ * 768 or 1024 threads (6, 10 or 14 rows of 62 cells); it is the default there,
+ * with the shape (also 2 rows) by the mesh's size, and schemes it does not cover
+ * run the stage kernels.  First-order steps with these fluxes are tiled there by
+ * default too (HLLC below about a million cells); a layout set for stage 0
+ * takes its place.  All choices give bit-identical results. */
 int zfv_set_launch(zfv_ctx* ctx, int stage, int layout, int block);
 int zfv_get_launch(zfv_ctx* ctx, int stage, int* layout, int* block);
 /* Schedule of the tiled step (layout 3): 0 (default) one workgroup per
- * tile; 1 persistent workgroups, as many as the GPU holds at once, each
+ * tile; 1 persistent workgroups (HLLC), as many as the GPU holds at once, each
  * walking the tiles of its XCD's range.  Results are bit-identical.  No
  * counterpart in the reference (its SmFluid::update loops over cells on the
  * CPU, sm_fluid.cpp:81-102). */
