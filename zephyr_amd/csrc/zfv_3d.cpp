@@ -44,9 +44,10 @@ inline double smin_h(double a, double b) { return (b < a) ? b : a; }
 
 constexpr int kSides = 6;      // L, R, B, T, Z (back), F (front)
 // States up to this size are downloaded through pinned memory that the kernel
-// writes: six copies to pageable memory behind a kernel cost 150 us for 13468
-// cells (125 without the kernel, when every field was an array of its own).
-constexpr size_t kHostRows = (size_t)1 << 20;
+// writes (us; six copies to pageable memory behind a kernel / so): 13468 cells
+// 152 / 81, 24000 188 / 105; against 349 and 622 with every field an array of its
+// own and no kernel, 110592 305, 166320 566.
+constexpr size_t kHostRows = (size_t)8 << 20;
 constexpr int kSlots24 = 24;   // AMR-3D face slots per cell (geom/indexing.h:340-372)
 
 }  // namespace
