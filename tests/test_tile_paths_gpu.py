@@ -110,6 +110,39 @@ def test_upload_keeps_the_last_steps_gradients(zfv):
         assert_same(ref.grad(), til.grad(), after)
 
 
+@pytest.mark.parametrize("flux", ["hllc", "hll", "rusanov"])
+@pytest.mark.parametrize("upload", [False, True])
+@pytest.mark.parametrize("graphs", [False, True])
+@pytest.mark.parametrize("then", ["limiter", "first order", "autotune", "first-order autotune", "refine"])
+def test_gradients_are_the_last_muscl_steps(zfv, flux, upload, graphs, then):
+    """grad() returns what the stage kernels stored in the last MUSCL step,
+    whatever is configured, stepped, timed or adapted before it is asked for."""
+    out = []
+    for ctx in pair(zfv, 30, 70, (2, 1, 3, 3), 2, flux):
+        ctx.graph_enable(graphs)
+        ctx.step(9)   # with graphs a replay of six steps and three more
+        if graphs:
+            ctx.step(6)   # a replay is the last
+        if upload:
+            ctx.set_state(*quadrants(30, 70, 12))
+        if then == "limiter":
+            ctx.configure(acc=2, flux=flux, limiter="minmod", cfl=0.5, gamma=GAMMA)
+        elif then == "first order":
+            ctx.configure(acc=1, flux=flux, limiter="MC", cfl=0.5, gamma=GAMMA)
+            ctx.step(7)
+        elif then == "autotune":   # its timed launches leave the gradients of the current state
+            ctx.autotune(reps=1)
+        elif then == "first-order autotune":
+            ctx.configure(acc=1, flux=flux, limiter="MC", cfl=0.5, gamma=GAMMA)
+            ctx.autotune(reps=1)
+        else:   # the slope distributor reads them
+            ctx.configure(acc=2, flux=flux, limiter="vanLeer", cfl=0.5, gamma=GAMMA)
+            ctx.set_flags_array(np.where(np.arange(30 * 70) % 17 < 4, 1, 0))
+            ctx.refine(1, slope=True)
+        out.append(ctx.state() if then == "refine" else ctx.grad())
+    equal(out[0], out[1], then)
+
+
 def test_gradients_after_graph_replays_and_batch_uploads(zfv):
     sizes = [(20, 33), (7, 62), (3, 3)]
     out = []

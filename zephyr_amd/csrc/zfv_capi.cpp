@@ -158,11 +158,14 @@ struct zfv_ctx {
     int tile_variant = 0;
     bool tile_persistent = false;   // tiled step by persistent workgroups (else one workgroup per tile)
     // The tiled step does not store its gradients: after one, the gradients
-    // of the last step are recomputed on demand from its input (layer 1 - cur).
+    // of the last step are recomputed on demand from its input (layer 1 - cur)
+    // with its limiter.
     bool grad_pending = false;
-    // ... with the limiter that was set when a state upload followed the step
-    // (-1: none did, the limiter set when they are asked for)
-    int grad_limiter = -1;
+    int grad_limiter = 0;
+    void defer_grads() {
+        grad_pending = true;
+        grad_limiter = prm.limiter;
+    }
     // dt and error word of a synchronising call, in pinned host memory
     struct Report {
         double dt;
@@ -1618,9 +1621,8 @@ static int state_upload(zfv_ctx* ctx, const double* const* src, hipMemcpyKind ki
     const int n = ctx->hm.n;
     for (int k = 0; k < 5; ++k)
         if (!src[k]) return fail(ZFV_ERR_ARG, "null state array");
-    // The last tiled step's gradients are recomputed on demand from its input,
-    // layer 1 - cur, whose cells an upload leaves as they are.
-    if (ctx->grad_pending && ctx->grad_limiter < 0) ctx->grad_limiter = ctx->prm.limiter;
+    // An upload leaves layer 1 - cur, from which the last tiled step's gradients
+    // may be recomputed, as it is (but for a batch's padding cells).
     double *dst[5], *dst2[5];
     for (int k = 0; k < 5; ++k) {
         dst[k] = ctx->st[ctx->cur][k].p;
@@ -1792,8 +1794,7 @@ static int step_once(zfv_ctx* ctx) {
                                     eos, ctl, ctx->stream);
         }));
         ctx->wcur = 1 - ctx->wcur;
-        ctx->grad_pending = true;   // the step's gradients were not stored
-        ctx->grad_limiter = -1;
+        ctx->defer_grads();
         ctx->co.grad = false;
     } else {
         DevGrad G{ctx->gdx.p, ctx->gdy.p};
@@ -1817,15 +1818,16 @@ static int step_once(zfv_ctx* ctx) {
     return ZFV_OK;
 }
 
-// The gradients of the last step, when a tiled step did not store them:
-// the gradient kernel on that step's input, layer 1 - cur (intact until the
-// next step or upload, before which this runs).
+// The gradients of the last MUSCL step, when a tiled step did not store them:
+// the gradient kernel on that step's input, layer 1 - cur.  That layer stays as
+// it is until the next step (a MUSCL step brings its own gradients; before any
+// other call that writes the layer this runs).
 static int materialize_grads(zfv_ctx* ctx) {
     if (!ctx->grad_pending) return ZFV_OK;
     const DevGrad G{ctx->gdx.p, ctx->gdy.p};
     const int prev = 1 - ctx->cur;
-    const int limiter = ctx->grad_limiter < 0 ? ctx->prm.limiter : ctx->grad_limiter;
-    ZFV_HIP(launch_grad_pred(limiter, false, ctx->gp_layout(), ctx->gp_block(), ctx->dmesh(), ctx->layer(prev), G, ctx->layer(2), ctx->wait[ctx->wcur].p, ctx->eos(), make_ctl(ctx),
+    ZFV_HIP(launch_grad_pred(ctx->grad_limiter, false, ctx->gp_layout(), ctx->gp_block(), ctx->dmesh(),
+                             ctx->layer(prev), G, ctx->layer(2), ctx->wait[ctx->wcur].p, ctx->eos(), make_ctl(ctx),
                              ctx->stream));
     ctx->grad_pending = false;
     ctx->co.grad = false;
@@ -1894,7 +1896,7 @@ int zfv_smf_step(zfv_ctx* ctx, int n_steps) {
     if (n_steps < 0) return fail(ZFV_ERR_ARG, "negative step count");
     r = to_curve_order(ctx);
     if (r) return r;
-    if (ctx->prm.acc == 1 && ctx->grad_limiter >= 0 && n_steps > 0) {
+    if (ctx->prm.acc == 1 && n_steps > 0) {
         r = materialize_grads(ctx);   // a first-order step overwrites their input and brings none
         if (r) return r;
     }
@@ -1908,10 +1910,7 @@ int zfv_smf_step(zfv_ctx* ctx, int n_steps) {
             if (r) return r;
             ZFV_HIP(hipGraphLaunch(exec, ctx->stream));
             ctx->step_no += kGraphSteps;   // cur and wcur return to their values after 6 swaps
-            if (ctx->tile_step()) {        // as step_once leaves them (a replay does not run it)
-                ctx->grad_pending = true;
-                ctx->grad_limiter = -1;
-            }
+            if (ctx->tile_step()) ctx->defer_grads();   // a replay does not run step_once
             it += kGraphSteps;
         }
     }
@@ -3223,6 +3222,8 @@ int zfv_autotune(zfv_ctx* ctx, int reps, double* ms_out) {
     if (r) return r;
     if (reps <= 0) return fail(ZFV_ERR_ARG, "reps must be positive");
     r = to_curve_order(ctx);   // tune on the order the steps will run in
+    if (r) return r;
+    r = materialize_grads(ctx);   // the timed launches write the layer they come from
     if (r) return r;
     r = ensure_dt(ctx);
     if (r) return r;
