@@ -1,0 +1,83 @@
+"""Host paths of libzfv.so that must hold when a call fails or is handed short
+buffers, on the CPU: libzfv.so over a stand-in for the HIP runtime
+(tests/hostshim/hip_stub.cpp), which checks copies against the allocations,
+records the launches without running them, and makes chosen calls fail."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes as C, sys
+import numpy as np
+hip = C.CDLL(sys.argv[1], C.RTLD_GLOBAL)
+hip.stub_launch.restype = C.c_char_p
+hip.stub_word.restype = C.c_uint64
+hip.stub_pinned.restype = C.c_size_t
+import zephyr_amd as Z
+
+def launches():
+    return [(hip.stub_launch(i).decode(), hip.stub_word(i)) for i in range(hip.stub_launches())]
+
+def fails(call):
+    try:
+        call()
+    except Z.ZfvError:
+        return True
+    return False
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    if shutil.which("g++") is None or not os.path.exists("/opt/rocm/include/hip/hip_runtime_api.h"):
+        pytest.skip("needs g++ and the HIP headers")
+    so = str(tmp_path_factory.mktemp("stub") / "libhipstub.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(ROOT, "tests", "hostshim", "hip_stub.cpp"), "-o", so], check=True)
+
+    def run(code):
+        out = subprocess.run([sys.executable, "-c", PRELUDE + code, so], capture_output=True, text=True, cwd=ROOT,
+                             timeout=120)
+        assert out.returncode == 0, out.stdout + out.stderr
+    return run
+
+
+@pytest.mark.parametrize("overlap,call,after", [
+    (0, "8k_mm_crpI", 0), (0, "10k_mm_flux1I", 0), (1, "10k_mm_flux1I", 0), (2, "8k_mm_crpI", 0),
+    (2, "hipStreamWaitEvent", 1), (2, "hipStreamWaitEvent", 2), (2, "15k_mm_take_count", 0)])
+def test_composite_face_counters_are_clear_after_a_failed_step(stub, overlap, call, after):
+    """Every marking starts from counters that nothing has appended to: taken
+    by the last step's update, or cleared after a step that failed between."""
+    stub(f"""
+ctx = Z.Context()
+ctx.mesh_rectangle(8, 8)
+ctx.mm_configure([(1.4, 0, 0, 718.0, 0, 1.2), (1.6, 0, 0, 3116.0, 0, 0.2)])
+ctx.mm_set_overlap({overlap})
+one = np.ones(64)
+ctx.mm_set_state(one, one, one, one, np.stack([one, 0 * one]))
+hip.stub_keep(b"10k_fill_u64", 0)
+hip.stub_keep(b"13k_mm_crp_markI", 8)
+ctx.mm_step(1)
+hip.stub_reset()
+ctx.mm_step(1)
+calls = launches()
+count = [w for name, w in calls if "k_mm_crp_mark" in name]
+assert len(count) == 1 and not any("k_fill_u64" in name for name, w in calls), calls   # the update takes them
+for attempt in range(2):
+    hip.stub_fail({call.encode()!r}, {after})
+    assert fails(lambda: ctx.mm_step(1))
+    hip.stub_reset()
+    if attempt:
+        ctx.mm_step(1)
+        calls = launches()
+        mark = [i for i, (name, w) in enumerate(calls) if "k_mm_crp_mark" in name][0]
+        assert any("k_fill_u64" in name and w == count[0] for name, w in calls[:mark]), calls
+hip.stub_reset()
+ctx.mm_step(1)
+assert not any("k_fill_u64" in name for name, w in launches())
+""")

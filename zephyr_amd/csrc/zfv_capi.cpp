@@ -227,6 +227,7 @@ struct zfv_ctx {
         int acc = 1;                  // m_acc (mm_fluid.h:157)
         DBuf<int> crp_list, crp_cells;
         DBuf<unsigned int> crp_count;   // [0] listed faces, [1] listed cells, [2] the last sweep's faces
+        bool crp_open = false;          // a marking was enqueued, and not the launch that takes its counters
         DBuf<unsigned long long> dtmin;
         // The composite fluxes on a second stream (same priority), beside
         // the update of the cells without a composite face: `side` and the
@@ -2638,6 +2639,14 @@ int zfv_mm_step(zfv_ctx* ctx, int n_steps) {
         if (S.crp_count.n != 4) {
             ZFV_HIP(S.crp_count.alloc(4));
             ZFV_HIP(launch_fill_u64((unsigned long long*)S.crp_count.p, 2, 0ULL, ctx->stream));
+            S.crp_open = false;
+        }
+        if (S.crp_open) {
+            // A call that failed after its marking left the counters; the next
+            // marking would append behind its faces and, repeated, past the list.
+            if (S.side) ZFV_HIP(hipStreamSynchronize(S.side));   // its composite fluxes may still read them
+            ZFV_HIP(launch_fill_u64((unsigned long long*)S.crp_count.p, 1, 0ULL, ctx->stream));
+            S.crp_open = false;
         }
         if (S.overlap) {
             if (S.overlap == 2 && S.crp_cells.n != cap) ZFV_HIP(S.crp_cells.alloc(cap));
@@ -2703,6 +2712,7 @@ int zfv_mm_step(zfv_ctx* ctx, int n_steps) {
                 }));
             }
             if (S.crp) {   // the composite fluxes of the sweep's faces
+                S.crp_open = true;
                 ZFV_HIP(timed(ctx, "mm_crp_mark", [&] {
                     return mm_crp_mark(M, in, half, S.mix, acc, o, S.gx.p, S.gy.p, S.crp_list.p,
                                        mode == 2 ? S.crp_cells.p : nullptr, S.crp_count.p,
@@ -2742,6 +2752,7 @@ int zfv_mm_step(zfv_ctx* ctx, int n_steps) {
                 ZFV_HIP(update(2));
                 ZFV_HIP(mm_take_count(S.crp_count.p, s1));
             }
+            S.crp_open = false;
             S.cur = 1 - S.cur;   // MmFluid::swap, after every integrate
         }
         S.step_no += 1;
