@@ -81,3 +81,50 @@ hip.stub_reset()
 ctx.mm_step(1)
 assert not any("k_fill_u64" in name for name, w in launches())
 """)
+
+
+@pytest.mark.parametrize("row", range(5))
+@pytest.mark.parametrize("short", [8, 8 * 35])
+def test_short_device_rows_are_refused(stub, row, short):
+    """A device row that ends before its last cell is refused, as by hipMemcpy,
+    and no kernel is given it; a row of exactly the mesh's cells, at the end of a
+    larger allocation, is copied by the kernel, one off an 8-byte boundary is not."""
+    stub(f"""
+n = 36
+ctx = Z.Context()
+ctx.mesh_rectangle(6, 6)
+ctx.configure()
+one = np.ones(n)
+ctx.set_state(one, one, one, one, one)
+
+def device(nbytes):
+    p = C.c_void_p()
+    assert hip.hipMalloc(C.byref(p), C.c_size_t(nbytes)) == 0
+    return p.value
+
+up, down = Z.lib().zfv_state_upload_device, Z.lib().zfv_state_download_device
+
+def go(call, rows):
+    hip.stub_reset()
+    code = call(ctx.h, *[C.c_void_p(p) for p in rows])
+    return code, any("k_state_copy" in name for name, w in launches())
+
+rows = [device(8 * n) for _ in range(5)]
+tail = device(8 * n + 16)
+for call in (up, down):
+    assert go(call, rows) == (0, True)
+    end = list(rows)
+    end[{row}] = tail + 16
+    assert go(call, end) == (0, True)
+    off = list(rows)
+    off[{row}] = tail + 4
+    assert go(call, off) == (0, False)
+    late = list(rows)
+    late[{row}] = tail + 24
+    code, kernel = go(call, late)
+    assert code == Z.ZFV_ERR_HIP and not kernel
+    less = list(rows)
+    less[{row}] = device(8 * n - {short})
+    code, kernel = go(call, less)
+    assert code == Z.ZFV_ERR_HIP and not kernel
+""")

@@ -1600,16 +1600,22 @@ int zfv_smf_set_max_dt(zfv_ctx* ctx, double max_dt) {
 
 static int materialize_grads(zfv_ctx* ctx);
 
-// Whether the five rows lie in this device's own memory, where one kernel can
-// copy them (other memory goes through hipMemcpy, as before).
-static bool on_device(const zfv_ctx* ctx, const double* const* rows) {
+// Whether the five rows lie in this device's own memory with all of their n
+// doubles, where one kernel can copy them.  Other memory goes through hipMemcpy,
+// which refuses a row that ends before its n-th double.
+static bool on_device(const zfv_ctx* ctx, const double* const* rows, int n) {
     for (int k = 0; k < 5; ++k) {
         hipPointerAttribute_t a;
-        if (hipPointerGetAttributes(&a, rows[k]) != hipSuccess) {
+        hipDeviceptr_t base = nullptr;
+        size_t size = 0;
+        if (hipPointerGetAttributes(&a, rows[k]) != hipSuccess || a.type != hipMemoryTypeDevice ||
+            a.device != ctx->device ||
+            hipMemGetAddressRange(&base, &size, const_cast<double*>(rows[k])) != hipSuccess) {
             (void)hipGetLastError();   // not a HIP allocation
             return false;
         }
-        if (a.type != hipMemoryTypeDevice || a.device != ctx->device) return false;
+        const uintptr_t p = (uintptr_t)rows[k], b = (uintptr_t)base;
+        if (p % sizeof(double) || p < b || p - b > size || (size - (p - b)) / sizeof(double) < (size_t)n) return false;
     }
     return true;
 }
@@ -1633,7 +1639,7 @@ static int state_upload(zfv_ctx* ctx, const double* const* src, hipMemcpyKind ki
     // both alternating layers the uploaded values there, so a download
     // returns them whatever the parity of the step count.
     const DevMesh M = ctx->dmesh();
-    if (kind == hipMemcpyDeviceToDevice && on_device(ctx, src)) {
+    if (kind == hipMemcpyDeviceToDevice && on_device(ctx, src, n)) {
         ZFV_HIP(launch_state_copy(src, dst, M.chunk_pid ? dst2 : nullptr, M, ctx->dtmin.p, 3 * ctx->nseg, nullptr,
                                   nullptr, ctx->stream));
         ctx->slots_reset = true;
@@ -1659,7 +1665,7 @@ static int state_download(zfv_ctx* ctx, double* const* dst, hipMemcpyKind kind) 
         if (!dst[k]) return fail(ZFV_ERR_ARG, "null state array");
     double* src[5];
     for (int k = 0; k < 5; ++k) src[k] = ctx->st[ctx->cur][k].p;
-    if (kind == hipMemcpyDeviceToDevice && on_device(ctx, dst)) {
+    if (kind == hipMemcpyDeviceToDevice && on_device(ctx, dst, n)) {
         ZFV_HIP(launch_state_copy(src, dst, nullptr, ctx->dmesh(), nullptr, 0, ctx->err.p, &ctx->report->err, ctx->stream));
     } else {
         for (int k = 0; k < 5; ++k)
