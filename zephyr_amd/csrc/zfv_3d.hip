@@ -597,11 +597,11 @@ __global__ void __launch_bounds__(256) k3_grad_pred(Dev3Mesh M, Dev3State in, do
 // CFL candidate of the new state.  The workgroup's cells leave their records in
 // LDS for the neighbours among them (all but a few along z, and along y while
 // nz < 256): with every neighbour read from memory the L1 cache was busy 89 % of
-// the time.  Three waves a SIMD, which spills two registers, since a wave waits
-// for loads 43 % of its time.  96^3 cells, HLLC: 165 us with one array a field
-// and no LDS, 137 with pairs, 119 so (133 at two waves); the vector instructions
-// alone take 87.  Evaluating each face once for both of its cells (tiles marched
-// along x) took 170: with 3D's larger state the exchange costs what it saves.
+// the time.  96^3 cells, HLLC: 165 us with one array a field and no LDS, 137 with
+// pairs, 119 so at three waves a SIMD (133 at two; a wave waits for loads 43 % of its
+// time); the vector instructions alone take 87.  Evaluating each face once for
+// both of its cells (tiles marched along x) took 170: with 3D's larger state the
+// exchange costs what it saves.
 template <int FLUX, bool TAB>
 __device__ __forceinline__ double corr_cell(const Dev3Mesh& M, const Dev3State& init, const double2* __restrict__ R,
                                             int* __restrict__ wait_out, const Dev3State& next, const Eos& eos,
@@ -675,9 +675,20 @@ __device__ __forceinline__ double corr_cell(const Dev3Mesh& M, const Dev3State& 
     return cell_dt3(zn, M.h[c], eos);
 }
 
+// Waves a SIMD that the corrector's registers are allocated for.  HLLC and its
+// variants spill 8 to 16 registers for the third one and gain by it; every other
+// flux would spill 52 to 160 (Rusanov none, at either), and on the slot arrays
+// HLLC 68.  At 96^3 with MC, two waves / three, us: tables HLLC 138 / 123, HLLC_M
+// 148 / 132, HLLC_LM 161 / 139, Rusanov 102 / 102, HLL 133 / 250, CIR1 205 / 240, CIR2
+// 179 / 186, Godunov 1094 / 1227; slot arrays HLLC 222 / 219 (61 x 83 x 95 112 / 118),
+// HLL 223 / 325, CIR1 279 / 334, Godunov 1134 / 1225.
 template <int FLUX, bool TAB>
-__global__ void __launch_bounds__(256, 3) k3_corr(Dev3Mesh M, Dev3State init, const double2* __restrict__ R,
-                                               int* __restrict__ wait_out, Dev3State next, Eos eos, Dev3Ctl ctl) {
+constexpr int kCorrWaves = TAB && FLUX >= 3 && FLUX <= 5 ? 3 : 2;
+
+template <int FLUX, bool TAB>
+__global__ void __launch_bounds__(256, (kCorrWaves<FLUX, TAB>)) k3_corr(
+    Dev3Mesh M, Dev3State init, const double2* __restrict__ R, int* __restrict__ wait_out, Dev3State next, Eos eos,
+    Dev3Ctl ctl) {
     const int c = cell_of_thread();
     const double dt = block_dt(ctl);
     step_epilogue0(ctl, dt);
