@@ -231,6 +231,9 @@ __device__ __forceinline__ Place place_of(const TileMesh& T, int b) {
     return p;
 }
 
+// Whether this lane has a top face: from_next gives the last one no state.
+__device__ __forceinline__ bool top_lane(const Place& p) { return p.l < 63; }
+
 __device__ __forceinline__ void tile_prologue(const StepCtl& ctl, const Place& p, double dt) {
     if (p.first && threadIdx.x == 0) {
         ctl.dt_out[p.pid] = dt;
@@ -444,7 +447,7 @@ __device__ __forceinline__ void tile_body(const TileMesh& T, const DevState& in,
             }
             bool nanA = false, nanB = false;
             Q FA, GB;
-            flux_pair_robust<FLUX>(top_local(A), top_local(B), rob, eos, nanA, nanB, FA, GB);
+            flux_pair_robust<FLUX>(top_local(A), top_local(B), rob, eos, top_lane(p), nanA, nanB, FA, GB);
             fT = scaled(top_global(FA), C.aT);
             fB = from_prev(scaled(top_global(GB), C.aB));
             bad |= (nanA && out_lane) || (nanB && p.l < kTileJ && p.gv + 1 < p.ny);
@@ -460,7 +463,7 @@ __device__ __forceinline__ void tile_body(const TileMesh& T, const DevState& in,
         if (p.gu == -1 && !p.perx) robR = wc > 0;
         bool nanA = false, nanB = false;
         Q FA, GB;
-        flux_pair_robust<FLUX>(A, B, robR, eos, nanA, nanB, FA, GB);
+        flux_pair_robust<FLUX>(A, B, robR, eos, true, nanA, nanB, FA, GB);
         fR = scaled(FA, R[kRowAR * 64]);
         const Q g = scaled(GB, R[kRowAL * 64]);
         ex[x + 64] = g.r;
@@ -532,7 +535,7 @@ __device__ __forceinline__ void tile_flux1_body(const TileMesh& T, const DevStat
         }
         bool nanA = false, nanB = false;
         Q FA, GB;
-        flux_pair<FLUX>(top_local(A), top_local(B), eos, nanA, nanB, FA, GB);
+        flux_pair<FLUX>(top_local(A), top_local(B), eos, top_lane(p), nanA, nanB, FA, GB);
         fT = scaled(top_global(FA), C.aT);
         fB = from_prev(scaled(top_global(GB), C.aB));
         bad |= (nanA && out_lane) || (nanB && p.l < kTileJ && p.gv + 1 < p.ny);
@@ -546,7 +549,7 @@ __device__ __forceinline__ void tile_flux1_body(const TileMesh& T, const DevStat
         }
         bool nanA = false, nanB = false;
         Q FA, GB;
-        flux_pair<FLUX>(A, B, eos, nanA, nanB, FA, GB);
+        flux_pair<FLUX>(A, B, eos, true, nanA, nanB, FA, GB);
         fR = scaled(FA, aR);
         const Q g = scaled(GB, aL);
         ex[x + 64] = g.r;
