@@ -435,9 +435,9 @@ int zfv_restore(zfv_ctx* ctx, const char* root);
  * one).  Layout 3 (stage 1 only) runs the whole MUSCL step with the HLLC, HLL
  * or Rusanov flux in one tiled kernel with the half states and gradients in
  * LDS, on meshes built by zfv_mesh_rectangle / zfv_batch_rectangles (before any
- * adaptation; ZFV_ERR_UNSUPPORTED otherwise); its block is the tile shape, 512,
- * 768 or 1024 threads (6, 10 or 14 rows of 62 cells); it is the default there,
- * with the shape (also 2 rows) by the mesh's size, and schemes it does not cover
+ * adaptation; ZFV_ERR_UNSUPPORTED otherwise); its block is the tile shape, 256,
+ * 512, 768 or 1024 threads (2, 6, 10 or 14 rows of 62 cells); it is the default
+ * there, with the shape by the mesh's size, and schemes it does not cover
  * run the stage kernels.  First-order steps with these fluxes are tiled there by
  * default too (HLLC below about a million cells); a layout set for stage 0
  * takes its place.  All choices give bit-identical results. */
@@ -458,7 +458,7 @@ int zfv_get_tile_schedule(zfv_ctx* ctx, int* persistent);
  * launch indexed [stage][layout 0-3][block 128/256/512, or for layout 3 the
  * tile shape 512/768/1024], where [1][3][shape] is the tiled step with one
  * workgroup per tile and [2][3][shape] with persistent workgroups (0 where
- * not timed). */
+ * not timed; the 256-thread shape is timed too and has no place here). */
 int zfv_autotune(zfv_ctx* ctx, int reps, double* ms_out);
 /* Capture steps into HIP graphs (6 steps per graph, one graph per starting
  * phase, replayed by zfv_smf_step; re-captured after any change of mesh,

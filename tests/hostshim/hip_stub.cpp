@@ -31,6 +31,9 @@ std::string fail_call;
 int fail_after = 0;
 hipError_t last_error = hipSuccess;
 size_t pinned_bytes = 0;
+std::map<std::string, float> cost;   // part of a kernel's name -> ms a launch takes (others 1)
+float clock_ms = 0.0f;
+std::map<hipEvent_t, float> events;
 
 // the block that holds p, or null
 const std::pair<const uintptr_t, Block>* block_of(const void* p) {
@@ -87,6 +90,7 @@ const char* stub_launch(int i) { return launches[i].name.c_str(); }
 void stub_keep(const char* kernel, int k) { keep[kernel] = k; }
 uint64_t stub_word(int i) { return launches[i].word; }
 size_t stub_pinned() { return pinned_bytes; }
+void stub_cost(const char* kernel, double ms) { cost[kernel] = (float)ms; }
 
 // ---- registration and launches
 void** __hipRegisterFatBinary(const void*) {
@@ -118,6 +122,10 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipSt
     for (const auto& kv : keep)
         if (l.name.find(kv.first) != std::string::npos) memcpy(&l.word, args[kv.second], sizeof(l.word));
     launches.push_back(l);
+    float ms = 1.0f;
+    for (const auto& kv : cost)
+        if (l.name.find(kv.first) != std::string::npos) ms = kv.second;
+    clock_ms += ms;
     return hipSuccess;
 }
 hipError_t hipGetLastError() {
@@ -195,11 +203,11 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return ok("hipStreamSynchronize"); }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return ok("hipStreamWaitEvent"); }
-hipError_t hipEventCreate(hipEvent_t* e) { *e = (hipEvent_t)&token; return ok("hipEventCreate"); }
+hipError_t hipEventCreate(hipEvent_t* e) { *e = (hipEvent_t)malloc(1); return ok("hipEventCreate"); }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
-hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return ok("hipEventRecord"); }
+hipError_t hipEventDestroy(hipEvent_t e) { events.erase(e); free(e); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { events[e] = clock_ms; return ok("hipEventRecord"); }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 1.0f; return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) { *ms = events[b] - events[a]; return hipSuccess; }
 
 }  // extern "C"

@@ -128,3 +128,43 @@ for call in (up, down):
     code, kernel = go(call, less)
     assert code == Z.ZFV_ERR_HIP and not kernel
 """)
+
+
+@pytest.mark.parametrize("rows,block", [(2, 256), (6, 512), (10, 768), (14, 1024)])
+def test_tile_shape_that_runs_is_reported_kept_and_tuned(stub, rows, block):
+    """launch() reports the shape the steps run, set_launch(1, TILE, 0) and
+    set_launch of what was reported keep it, and the autotuner takes the
+    fastest of all four."""
+    stub(f"""
+def make(nx, ny):
+    ctx = Z.Context()
+    ctx.mesh_rectangle(nx, ny)
+    ctx.configure(acc=2, flux="hllc", limiter="MC")
+    one = np.ones(nx * ny)
+    ctx.set_state(one, one, one, one, one)
+    return ctx
+
+def runs(ctx):
+    hip.stub_reset()
+    ctx.step(1)
+    name = [n for n, w in launches() if "k_tile_step" in n][-1]
+    return (int(name.split("ELi")[3].split("E")[0]) + 2) * 64
+
+seen = set()
+for nx, ny in ((8, 8), (64, 48), (200, 200), (330, 280), (520, 390), (900, 700)):
+    ctx = make(nx, ny)
+    shape = runs(ctx)
+    seen.add(shape)
+    assert ctx.launch(1) == (Z.TILE, shape), (nx, ny, ctx.launch(1), shape)
+    ctx.set_launch(1, Z.TILE, 0)
+    assert runs(ctx) == shape and ctx.launch(1) == (Z.TILE, shape)
+    ctx.set_launch(1, Z.TILE, {block})
+    assert runs(ctx) == {block} and ctx.launch(1) == (Z.TILE, {block})
+assert 256 in seen and len(seen) > 1, seen
+ctx = make(64, 48)
+hip.stub_cost(b"k_tile_stepILi3ELi3E", C.c_double(0.5))
+hip.stub_cost(b"k_tile_stepILi3ELi3ELi{(6, 10, 14, 2).index(rows)}ELi{rows}E", C.c_double(0.25))
+ms = ctx.autotune(reps=2)
+assert ctx.launch(1) == (Z.TILE, {block}) and runs(ctx) == {block}
+assert np.all(ms[1, 3] == [0.25 if r == {rows} else 0.5 for r in (6, 10, 14)]), ms[1, 3]
+""")

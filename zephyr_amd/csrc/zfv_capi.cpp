@@ -1744,8 +1744,7 @@ constexpr int kCus = 256;   // compute units of the MI355X
 // 9.5, 16, 20, 25 at k = 1 to 4, 6 rows 14, 25, 35, 46, 10 rows 19, 38, 14 rows
 // 23, 48; first order 2 rows 8.3, 13, 16, 19, 6 rows 12, 19, 22, 10 rows 14, 24,
 // 14 rows 16, 28.
-static int tile_shape(const zfv_ctx* ctx, double* cost = nullptr) {
-    const bool muscl = ctx->prm.acc == 2;
+static int tile_shape(const zfv_ctx* ctx, bool muscl, double* cost = nullptr) {
     if (ctx->layout_set[1] && muscl) return ctx->tile_variant;
     static const double a2[kTileVariants] = {5.5, 1.5, -3.0, 5.5}, b2[kTileVariants] = {10.0, 18.5, 26.0, 4.9};
     static const double a1[kTileVariants] = {7.0, 5.5, 4.0, 6.0}, b1[kTileVariants] = {5.2, 9.2, 12.4, 3.4};
@@ -1771,7 +1770,7 @@ static bool tile_first(const zfv_ctx* ctx) {
     if (!ctx->tile_covers() || ctx->prm.acc != 1 || !ctx->flux1_tile) return false;
     if (ctx->prm.flux != ZFV_HLLC) return true;
     double cost = 0.0;
-    (void)tile_shape(ctx, &cost);
+    (void)tile_shape(ctx, false, &cost);
     return cost < 13.0 + 53.0e-6 * ctx->hm.n;
 }
 
@@ -1786,7 +1785,7 @@ static int step_once(zfv_ctx* ctx) {
     DevState in = ctx->layer(ctx->cur), out = ctx->layer(nxt);
     if (tile_first(ctx)) {
         ZFV_HIP(timed(ctx, "flux1", [&] {
-            return launch_tile_flux1(P.flux, tile_shape(ctx), ctx->tmesh(), in, out, eos, ctl, ctx->stream);
+            return launch_tile_flux1(P.flux, tile_shape(ctx, false), ctx->tmesh(), in, out, eos, ctl, ctx->stream);
         }));
     } else if (P.acc == 1) {
         ZFV_HIP(timed(ctx, "flux1", [&] {
@@ -1797,7 +1796,7 @@ static int step_once(zfv_ctx* ctx) {
         int* w_out = ctx->wait[1 - ctx->wcur].p;
         const TileMesh T = ctx->tmesh();
         ZFV_HIP(timed(ctx, "tile", [&] {
-            return launch_tile_step(P.flux, P.limiter, tile_shape(ctx), ctx->tile_persistent, T, in, out, w_in, w_out,
+            return launch_tile_step(P.flux, P.limiter, tile_shape(ctx, true), ctx->tile_persistent, T, in, out, w_in, w_out,
                                     eos, ctl, ctx->stream);
         }));
         ctx->wcur = 1 - ctx->wcur;
@@ -3169,7 +3168,7 @@ int zfv_limiter_from_name(const char* orig) {
 static bool valid_block(int b) { return b == 128 || b == 256 || b == 512; }
 
 static int tile_variant_of(int threads) {
-    for (int v = 0; v < kTileShapes; ++v)
+    for (int v = 0; v < kTileVariants; ++v)
         if (threads == (kTileRows[v] + 2) * 64) return v;
     return -1;
 }
@@ -3182,8 +3181,8 @@ int zfv_set_launch(zfv_ctx* ctx, int stage, int layout, int block) {
         if (stage != 1) return fail(ZFV_ERR_ARG, "the tiled layout is a stage-1 layout (it runs the whole step)");
         if (!ctx->have_mesh || !ctx->tiles.ok)
             return fail(ZFV_ERR_UNSUPPORTED, "the tiled layout needs a Rectangle mesh (or a batch of them)");
-        const int v = block == 0 ? ctx->tile_variant : tile_variant_of(block);
-        if (v < 0) return fail(ZFV_ERR_ARG, "tiled layout: block must be 0 (keep), 512, 768 or 1024");
+        const int v = block == 0 ? tile_shape(ctx, true) : tile_variant_of(block);
+        if (v < 0) return fail(ZFV_ERR_ARG, "tiled layout: block must be 0 (keep), 256, 512, 768 or 1024");
         ctx->layout[1] = kLayoutTile;
         ctx->block[1] = (kTileRows[v] + 2) * 64;
         ctx->tile_variant = v;
@@ -3225,7 +3224,11 @@ int zfv_get_launch(zfv_ctx* ctx, int stage, int* layout, int* block) {
     if (r) return r;
     if (stage < 0 || stage > 2) return fail(ZFV_ERR_ARG, "bad stage");
     if (layout) *layout = ctx->layout[stage];
-    if (block) *block = ctx->block[stage];
+    if (block) {
+        *block = ctx->block[stage];
+        if (stage == 1 && ctx->layout[1] == kLayoutTile && ctx->have_mesh && ctx->tiles.ok)
+            *block = (kTileRows[tile_shape(ctx, true)] + 2) * 64;   // the shape the steps run
+    }
     return ZFV_OK;
 }
 
@@ -3301,7 +3304,7 @@ int zfv_autotune(zfv_ctx* ctx, int reps, double* ms_out) {
         ctx->layout_set[st] = true;
         if (st == 0 && ctx->tile_covers()) {   // the tiled first-order step against the best layout
             const TileMesh T = ctx->tmesh();
-            const int v = tile_shape(ctx);
+            const int v = tile_shape(ctx, false);
             double ms = 0.0;
             r = time_it([&] { return launch_tile_flux1(P.flux, v, T, in, out, eos, ctl, s); }, ms);
             if (r) return r;
@@ -3311,22 +3314,25 @@ int zfv_autotune(zfv_ctx* ctx, int reps, double* ms_out) {
     // the tiled step (one kernel for the whole step) against the best pair
     // of gradient and corrector kernels
     if (P.acc == 2 && ctx->tile_covers()) {
-        // [1][tile][v]: one workgroup per tile; [2][tile][v]: persistent workgroups
+        // one workgroup per tile, then persistent workgroups; the first three
+        // shapes are reported as [1][tile][v] and [2][tile][v]
         const TileMesh T = ctx->tmesh();
+        double tt[2][kTileVariants] = {};
         int bv = 0, bp = 0;
         for (int pers = 0; pers < (P.flux == ZFV_HLLC ? 2 : 1); ++pers)
-            for (int v = 0; v < kTileShapes; ++v) {
+            for (int v = 0; v < kTileVariants; ++v) {
                 r = time_it([&] { return launch_tile_step(P.flux, P.limiter, v, pers != 0, T, in, out, w_in, w_out, eos, ctl, s); },
-                            t[1 + pers][kLayoutTile][v]);
+                            tt[pers][v]);
                 if (r) return r;
-                if (t[1 + pers][kLayoutTile][v] < t[1 + bp][kLayoutTile][bv]) {
+                if (v < 3) t[1 + pers][kLayoutTile][v] = tt[pers][v];
+                if (tt[pers][v] < tt[bp][bv]) {
                     bv = v;
                     bp = pers;
                 }
             }
         const double split = t[1][ctx->layout[1]][ctx->block[1] == 128 ? 0 : (ctx->block[1] == 256 ? 1 : 2)] +
                              t[2][ctx->layout[2]][ctx->block[2] == 128 ? 0 : (ctx->block[2] == 256 ? 1 : 2)];
-        if (t[1 + bp][kLayoutTile][bv] < split) {
+        if (tt[bp][bv] < split) {
             ctx->layout[1] = kLayoutTile;
             ctx->block[1] = (kTileRows[bv] + 2) * 64;
             ctx->tile_variant = bv;

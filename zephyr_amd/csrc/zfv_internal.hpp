@@ -219,10 +219,9 @@ enum TileRowQuantity {
 };
 // Tile shapes: kTileJ output cells along j (64-lane wavefronts with a halo
 // lane on each side) by kTileRows[v] along i, with (rows + 2) wavefronts
-// per workgroup (one per row of the tile and its two halo rows).  The first
-// kTileShapes can be chosen by the caller.
+// per workgroup (one per row of the tile and its two halo rows).
 constexpr int kTileJ = 62;
-constexpr int kTileVariants = 4, kTileShapes = 3;
+constexpr int kTileVariants = 4;
 constexpr int kTileRows[kTileVariants] = {6, 10, 14, 2};
 struct TileProb {
     int off, nx, ny;     // first cell, columns, rows
