@@ -437,10 +437,11 @@ int zfv_restore(zfv_ctx* ctx, const char* root);
  * LDS, on meshes built by zfv_mesh_rectangle / zfv_batch_rectangles (before any
  * adaptation; ZFV_ERR_UNSUPPORTED otherwise); its block is the tile shape, 256,
  * 512, 768 or 1024 threads (2, 6, 10 or 14 rows of 62 cells); it is the default
- * there, with the shape by the mesh's size, and schemes it does not cover
- * run the stage kernels.  First-order steps with these fluxes are tiled there by
- * default too (HLLC below about a million cells); a layout set for stage 0
- * takes its place.  All choices give bit-identical results. */
+ * there, with the shape by the mesh's size, but for narrow meshes (a few cells
+ * along j), where layout 0 takes less, and schemes it does not cover run the
+ * stage kernels.  First-order steps with these fluxes are tiled there by default
+ * too, by the same rule; a layout set for stage 0 takes its place.  All choices
+ * give bit-identical results. */
 int zfv_set_launch(zfv_ctx* ctx, int stage, int layout, int block);
 int zfv_get_launch(zfv_ctx* ctx, int stage, int* layout, int* block);
 /* Schedule of the tiled step (layout 3): 0 (default) one workgroup per

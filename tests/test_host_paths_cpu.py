@@ -168,3 +168,35 @@ ms = ctx.autotune(reps=2)
 assert ctx.launch(1) == (Z.TILE, {block}) and runs(ctx) == {block}
 assert np.all(ms[1, 3] == [0.25 if r == {rows} else 0.5 for r in (6, 10, 14)]), ms[1, 3]
 """)
+
+
+@pytest.mark.parametrize("flux", ["hllc", "hll", "rusanov"])
+def test_narrow_meshes_run_the_cell_kernels(stub, flux):
+    """The tiled steps run where they take less than one thread per cell: not on
+    meshes of a few cells along j, whose tiles are mostly lanes without a cell; a
+    caller's choice stands."""
+    stub(f"""
+def runs(ctx):
+    hip.stub_reset()
+    ctx.step(1)
+    return any("k_tile" in n for n, w in launches())
+
+for acc in (1, 2):
+    for nx, ny, tiled in ((10000, 1, False), (100000, 1, False), (50000, 4, False), (20000, 10, False), (5000, 4, False),
+                          (8, 8, True), (1, 1000, True), (64, 48, True), (4, 5000, True), (300, 200, True),
+                          (900, 700, True)):
+        ctx = Z.Context()
+        ctx.mesh_rectangle(nx, ny)
+        ctx.configure(acc=acc, flux={flux!r}, limiter="MC")
+        one = np.ones(nx * ny)
+        ctx.set_state(one, one, one, one, one)
+        assert runs(ctx) == tiled, (acc, nx, ny)
+        if acc == 2:
+            assert (ctx.launch(1)[0] == Z.TILE) == tiled
+            ctx.set_launch(1, Z.TILE, 0)
+            assert runs(ctx) and ctx.launch(1)[0] == Z.TILE
+            ctx.set_launch(1, Z.CELL, 256)
+        else:
+            ctx.set_launch(0, Z.CELL, 256)
+        assert not runs(ctx)
+""")

@@ -89,6 +89,8 @@ struct KernelTimer {
 
 }  // namespace
 
+static bool tile_pays(const zfv_ctx* ctx, bool muscl);
+
 struct zfv_ctx {
     int device = 0;
     hipStream_t own_stream = nullptr;
@@ -173,7 +175,7 @@ struct zfv_ctx {
     };
     Report* report = nullptr;
     bool slots_reset = false;   // the CFL slots hold +inf (state upload)
-    bool flux1_tile = true;     // first-order steps may run the tiled kernel (no layout was chosen for them)
+    int flux1_tile = -1;        // first-order steps on the tiled kernel: -1 where it pays, else no (0) or yes (1)
 
     // batch of independent problems (nseg > 1): padded cell offsets, valid
     // cell counts, device tables of the kernels' Tile lookup
@@ -342,7 +344,9 @@ struct zfv_ctx {
         return tiles.ok && tiles.shared && tile_flux_built(prm.flux) && !co.state && !prm.axial;
     }
     // ... and the MUSCL step runs it.
-    bool tile_step() const { return tile_covers() && prm.acc == 2 && layout[1] == kLayoutTile; }
+    bool tile_step() const {
+        return tile_covers() && prm.acc == 2 && layout[1] == kLayoutTile && (layout_set[1] || tile_pays(this, true));
+    }
     // Launch configuration of the gradient kernel when it runs on its own.
     int gp_layout() const { return layout[1] == kLayoutTile ? kLayoutCell : layout[1]; }
     int gp_block() const { return layout[1] == kLayoutTile ? kBlock : block[1]; }
@@ -1737,41 +1741,57 @@ int zfv_grad_download(zfv_ctx* ctx, double* dx, double* dy) {
 
 constexpr int kCus = 256;   // compute units of the MI355X
 
-// Tile shape of the steps: the caller's or the autotuner's, else the one
-// whose workgroups load the fullest CU least: k workgroups on a CU take about
-// a + b k us of a step.  Few rows per tile spread a small mesh over more CUs,
-// many rows compute fewer halo rows.  Measured (MUSCL, HLLC, MC; us): 2 rows
-// 9.5, 16, 20, 25 at k = 1 to 4, 6 rows 14, 25, 35, 46, 10 rows 19, 38, 14 rows
-// 23, 48; first order 2 rows 8.3, 13, 16, 19, 6 rows 12, 19, 22, 10 rows 14, 24,
-// 14 rows 16, 28.
-static int tile_shape(const zfv_ctx* ctx, bool muscl, double* cost = nullptr) {
-    if (ctx->layout_set[1] && muscl) return ctx->tile_variant;
-    static const double a2[kTileVariants] = {5.5, 1.5, -3.0, 5.5}, b2[kTileVariants] = {10.0, 18.5, 26.0, 4.9};
-    static const double a1[kTileVariants] = {7.0, 5.5, 4.0, 6.0}, b1[kTileVariants] = {5.2, 9.2, 12.4, 3.4};
-    const double *a = muscl ? a2 : a1, *b = muscl ? b2 : b1;
+// What a tiled step of the shape v is expected to take, us: k workgroups on the
+// fullest CU take about a + b k, HLL and Rusanov less of it.  Few rows per tile
+// spread a small mesh over more CUs, many rows compute fewer halo rows.  Measured
+// (back to back, HLLC; MUSCL with MC): 2 rows 10.5, 16, 19.5, 21.7 at k = 1 to 4, 36
+// at 8, 169 at 46; 6 rows 15, 22, 30, 39 at 1 to 4, 100 at 12, 131 at 16; 10 rows 18,
+// 34, 50, 65 at 1 to 4, 155 at 10; 14 rows 22, 43, 64 at 1 to 3, 143 at 7.  First
+// order: 2 rows 6, 10.5, 13.8, 15.2 at 1 to 4, 27 at 8; 6 rows 8, 13, 16.5, 20 at 1 to
+// 4, 66 at 16; 10 rows 10, 19, 26, 33 at 1 to 4; 14 rows 12, 22, 32 at 1 to 3, 69 at 7.
+// HLL takes 0.83 to 0.96 of these, Rusanov 0.8 to 0.9.
+static double tile_cost(const zfv_ctx* ctx, bool muscl, int v) {
+    static const double a2[kTileVariants] = {7.0, 3.6, 3.0, 7.7}, b2[kTileVariants] = {7.7, 15.2, 20.0, 3.7};
+    static const double a1[kTileVariants] = {5.0, 4.0, 2.8, 4.0}, b1[kTileVariants] = {3.8, 7.1, 9.5, 3.0};
+    const int flux = ctx->prm.flux, k = (ctx->tiles.n_tiles[v] + kCus - 1) / kCus;
+    const double share = flux == ZFV_HLL ? (muscl ? 0.88 : 0.83) : flux == ZFV_RUSANOV ? (muscl ? 0.86 : 0.8) : 1.0;
+    return share * (muscl ? a2[v] + b2[v] * k : a1[v] + b1[v] * k);
+}
+
+static int least_tile(const zfv_ctx* ctx, bool muscl) {
     int best = 0;
-    double least = 0.0;
-    for (int v = 0; v < kTileVariants; ++v) {
-        const double t = a[v] + b[v] * ((ctx->tiles.n_tiles[v] + kCus - 1) / kCus);
-        if (v == 0 || t < least) {
-            best = v;
-            least = t;
-        }
-    }
-    if (cost) *cost = least;
+    for (int v = 1; v < kTileVariants; ++v)
+        if (tile_cost(ctx, muscl, v) < tile_cost(ctx, muscl, best)) best = v;
     return best;
 }
 
-// Whether a first-order step runs the tiled kernel.  Rusanov and HLL always
-// (at 1361 x 1023 58 us against 79); HLLC, whose faces keep more registers,
-// up to the size from where the one-thread-per-cell kernel, about 13 us +
-// 53 us per million cells, is the faster one (1 M cells: 66 us against 76).
+// Tile shape of the steps: the caller's or the autotuner's, else the one that is
+// expected to take the least.
+static int tile_shape(const zfv_ctx* ctx, bool muscl) {
+    return ctx->layout_set[1] && muscl ? ctx->tile_variant : least_tile(ctx, muscl);
+}
+
+// Whether the tiled step is expected to take less than the one-thread-per-cell
+// kernels, about 18 us + 180 us per million cells for a MUSCL step (measured 20 at
+// 16 k cells, 50 at 200 k, 269 at 1.39 M) and 7.5 + 51 for a first-order one (HLLC 8.5,
+// 19.7, 77; a little less for HLL, and for Rusanov on small meshes).  It is but for
+// narrow meshes, of few cells along j, and batches of small ones, whose tiles
+// are mostly lanes without a cell (HLL, tiled / by cells, us: 10000 x 1 54 / 19, 50000 x 4
+// 220 / 50, 1000 problems of 20 x 20 124 / 82; first order 50000 x 4 98 / 18, 10000 x 63
+// 49 / 40, 256 of 64 x 64 77 / 49; and 4 x 50000 34 / 56, 17 / 20).
+static bool tile_pays(const zfv_ctx* ctx, bool muscl) {
+    const double cells = 1.0e-6 * ctx->hm.n;
+    const double by_cells = muscl                          ? 18.0 + 180.0 * cells
+                            : ctx->prm.flux == ZFV_RUSANOV ? 6.3 + 55.0 * cells
+                            : ctx->prm.flux == ZFV_HLL     ? 7.2 + 49.0 * cells
+                                                           : 7.5 + 51.0 * cells;
+    return tile_cost(ctx, muscl, least_tile(ctx, muscl)) < by_cells;
+}
+
+// Whether a first-order step runs the tiled kernel.
 static bool tile_first(const zfv_ctx* ctx) {
-    if (!ctx->tile_covers() || ctx->prm.acc != 1 || !ctx->flux1_tile) return false;
-    if (ctx->prm.flux != ZFV_HLLC) return true;
-    double cost = 0.0;
-    (void)tile_shape(ctx, false, &cost);
-    return cost < 13.0 + 53.0e-6 * ctx->hm.n;
+    if (!ctx->tile_covers() || ctx->prm.acc != 1) return false;
+    return ctx->flux1_tile < 0 ? tile_pays(ctx, false) : ctx->flux1_tile != 0;
 }
 
 // SmFluid::update x n_steps (sm_fluid.cpp:81-102).
@@ -3197,7 +3217,7 @@ int zfv_set_launch(zfv_ctx* ctx, int stage, int layout, int block) {
     ctx->layout[stage] = layout;
     if (block) ctx->block[stage] = block;
     ctx->layout_set[stage] = true;
-    if (stage == 0) ctx->flux1_tile = false;
+    if (stage == 0) ctx->flux1_tile = 0;
     ctx->graphs_clear();
     return ZFV_OK;
 }
@@ -3224,10 +3244,11 @@ int zfv_get_launch(zfv_ctx* ctx, int stage, int* layout, int* block) {
     if (r) return r;
     if (stage < 0 || stage > 2) return fail(ZFV_ERR_ARG, "bad stage");
     if (layout) *layout = ctx->layout[stage];
-    if (block) {
-        *block = ctx->block[stage];
-        if (stage == 1 && ctx->layout[1] == kLayoutTile && ctx->have_mesh && ctx->tiles.ok)
-            *block = (kTileRows[tile_shape(ctx, true)] + 2) * 64;   // the shape the steps run
+    if (block) *block = ctx->block[stage];
+    if (stage == 1 && ctx->layout[1] == kLayoutTile && ctx->have_mesh && ctx->tiles.ok) {   // what the steps run
+        const bool tile = ctx->layout_set[1] || tile_pays(ctx, true);
+        if (layout) *layout = tile ? kLayoutTile : kLayoutCell;
+        if (block) *block = tile ? (kTileRows[tile_shape(ctx, true)] + 2) * 64 : kBlock;
     }
     return ZFV_OK;
 }
@@ -3308,7 +3329,7 @@ int zfv_autotune(zfv_ctx* ctx, int reps, double* ms_out) {
             double ms = 0.0;
             r = time_it([&] { return launch_tile_flux1(P.flux, v, T, in, out, eos, ctl, s); }, ms);
             if (r) return r;
-            ctx->flux1_tile = ms < t[0][bl][bb];
+            ctx->flux1_tile = ms < t[0][bl][bb] ? 1 : 0;
         }
     }
     // the tiled step (one kernel for the whole step) against the best pair
