@@ -33,6 +33,7 @@ hipError_t last_error = hipSuccess;
 size_t pinned_bytes = 0;
 std::map<std::string, float> cost;   // part of a kernel's name -> ms a launch takes (others 1)
 float clock_ms = 0.0f;
+int copies = 0;
 std::map<hipEvent_t, float> events;
 
 // the block that holds p, or null
@@ -66,6 +67,7 @@ hipError_t give(void* p) {
 }
 hipError_t copy(void* d, const void* s, size_t bytes) {
     if (!fits(d, bytes) || !fits(s, bytes)) return hipErrorInvalidValue;
+    ++copies;
     memmove(d, s, bytes);
     return hipSuccess;
 }
@@ -90,6 +92,7 @@ const char* stub_launch(int i) { return launches[i].name.c_str(); }
 void stub_keep(const char* kernel, int k) { keep[kernel] = k; }
 uint64_t stub_word(int i) { return launches[i].word; }
 size_t stub_pinned() { return pinned_bytes; }
+int stub_copies() { return copies; }   // copies that went through the runtime so far
 void stub_cost(const char* kernel, double ms) { cost[kernel] = (float)ms; }
 
 // ---- registration and launches

@@ -200,3 +200,14 @@ for acc in (1, 2):
             ctx.set_launch(0, Z.CELL, 256)
         assert not runs(ctx)
 """)
+
+
+def test_tile_tables_of_a_mesh_are_three_copies(stub):
+    """A Rectangle's mesh upload copies its tile tables (problems, columns, rows)
+    in one copy each, beside the 22 of the mesh arrays."""
+    stub("""
+ctx = Z.Context()
+before = hip.stub_copies()
+ctx.mesh_rectangle(5, 7)
+assert hip.stub_copies() - before == 25, hip.stub_copies() - before
+""")

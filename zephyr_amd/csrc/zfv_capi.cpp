@@ -462,6 +462,7 @@ bool build_tiles(zfv_ctx* ctx, const std::vector<int>& code, const std::vector<d
         for (int i = 0; i < nx; ++i)
             for (int j = 0; j < ny; ++j) {
                 const size_t c = (size_t)off + (size_t)i * ny + j, f = 8 * c;
+                const Side &Ci = C[i], &Rj = Rw[j];
                 const int ts[4] = {i > 0 ? (int)SC_INNER : P.t[0], i < nx - 1 ? (int)SC_INNER : P.t[1],
                                    j > 0 ? (int)SC_INNER : P.t[2], j < ny - 1 ? (int)SC_INNER : P.t[3]};
                 const int want_code = ts[0] | (ts[1] << 4) | (ts[2] << 8) | (ts[3] << 12);
@@ -477,11 +478,11 @@ bool build_tiles(zfv_ctx* ctx, const std::vector<int>& code, const std::vector<d
                                     nb_t ? off + i * ny + (j + 1) % ny : self};
                 for (int sl = 0; sl < 4; ++sl)
                     if (m.adj[f + sl] != adj[sl]) return false;
-                if (m.cx[c] != C[i].cx || m.cy[c] != Rw[j].cy) return false;
-                const double ar[4] = {Rw[j].a[0], Rw[j].a[1], C[i].a[2], C[i].a[3]};
-                const double wt[4] = {C[i].w[0], C[i].w[1], Rw[j].w[2], Rw[j].w[3]};
+                if (m.cx[c] != Ci.cx || m.cy[c] != Rj.cy) return false;
+                const double ar[4] = {Rj.a[0], Rj.a[1], Ci.a[2], Ci.a[3]};
+                const double wt[4] = {Ci.w[0], Ci.w[1], Rj.w[2], Rj.w[3]};
                 for (int sl = 0; sl < 4; ++sl) {
-                    if (m.fcx[f + sl] != C[i].fx[sl] || m.fcy[f + sl] != Rw[j].fy[sl] || m.area[f + sl] != ar[sl])
+                    if (m.fcx[f + sl] != Ci.fx[sl] || m.fcy[f + sl] != Rj.fy[sl] || m.area[f + sl] != ar[sl])
                         return false;
                     if (w[(size_t)sl * n + c] != wt[sl]) return false;
                 }
@@ -530,16 +531,16 @@ bool build_tiles(zfv_ctx* ctx, const std::vector<int>& code, const std::vector<d
     }
     hipStream_t s = ctx->stream;
     const size_t nr = rows[0].size();
+    std::vector<double> row;   // one copy: twelve small ones took 25 us
+    row.reserve(kTileRowAll * nr);
+    for (const auto& q : rows) row.insert(row.end(), q.begin(), q.end());
     if (T.prob.alloc(probs.size()) != hipSuccess || T.col.alloc(cols.size()) != hipSuccess ||
-        T.row.alloc(kTileRowAll * nr) != hipSuccess)
+        T.row.alloc(row.size()) != hipSuccess)
         return false;
     if (hipMemcpyAsync(T.prob.p, probs.data(), probs.size() * sizeof(TileProb), hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(T.col.p, cols.data(), cols.size() * sizeof(TileCol), hipMemcpyHostToDevice, s) != hipSuccess)
+        hipMemcpyAsync(T.col.p, cols.data(), cols.size() * sizeof(TileCol), hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipMemcpyAsync(T.row.p, row.data(), row.size() * sizeof(double), hipMemcpyHostToDevice, s) != hipSuccess)
         return false;
-    for (int q = 0; q < kTileRowAll; ++q)
-        if (hipMemcpyAsync(T.row.p + q * nr, rows[q].data(), nr * sizeof(double), hipMemcpyHostToDevice, s) !=
-            hipSuccess)
-            return false;
     if (hipStreamSynchronize(s) != hipSuccess) return false;   // the host tables end here
     T.n_probs = (int)probs.size();
     T.n_rows = (int)nr;
