@@ -524,9 +524,12 @@ int zfv3_state_upload(zfv3_ctx* ctx, const double* rho, const double* u, const d
     }
     const double* src[6] = {rho, u, v, w, p, e};
     Z3HIP(hipStreamSynchronize(ctx->stream));
+    // on the kernel's stream: from device memory a copy on another one returns
+    // before it is done, and the kernel would not wait for it
     for (int k = 0; k < 6; ++k)
-        Z3HIP(hipMemcpy(ctx->staging() + k * N, src[k], N * sizeof(double), hipMemcpyHostToDevice));
+        Z3HIP(hipMemcpyAsync(ctx->staging() + k * N, src[k], N * sizeof(double), hipMemcpyDefault, ctx->stream));
     Z3HIP(launch3_pack(ctx->staging(), ctx->state(ctx->zi), ctx->stream));
+    Z3HIP(hipStreamSynchronize(ctx->stream));   // the arrays are the caller's again
     ctx->have_state = true;
     return state_changed(ctx);
 }
