@@ -211,3 +211,45 @@ before = hip.stub_copies()
 ctx.mesh_rectangle(5, 7)
 assert hip.stub_copies() - before == 25, hip.stub_copies() - before
 """)
+
+
+def test_3d_transfers_hold_little_pinned_memory(stub):
+    """A 3D context holds the pinned memory its largest transfer needs, at most two
+    parts of 2 MiB, until it is closed; without pinned memory or events the
+    arrays are copied as they are."""
+    stub("""
+base = hip.stub_pinned()
+
+def make(n):
+    ctx = Z.Context3()
+    ctx.mesh_cuboid(1, 1, n)
+    ctx.configure()
+    one = np.ones(n)
+    return ctx, lambda: ctx.set_state(one, one, one, one, one, one)
+
+ctx, up = make(1)
+up()
+ctx.state()
+assert hip.stub_pinned() - base == 48, hip.stub_pinned() - base
+ctx.grad()
+assert hip.stub_pinned() - base == 120
+ctx.close()
+assert hip.stub_pinned() == base
+ctx, up = make(200000)
+up()
+ctx.state()
+ctx.grad()
+assert hip.stub_pinned() - base <= 4 << 20
+ctx.close()
+assert hip.stub_pinned() == base
+for call in ("hipHostMalloc", "hipEventCreate"):
+    ctx, up = make(50000)
+    for transfer in (up, ctx.state, ctx.grad):
+        hip.stub_fail(call.encode(), 0)
+        before = hip.stub_copies()
+        transfer()
+        if transfer is up:   # one that failed to have it copies, the next has it
+            assert hip.stub_copies() - before >= 6
+    ctx.close()
+assert hip.stub_pinned() == base
+""")

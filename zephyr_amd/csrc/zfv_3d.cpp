@@ -8,6 +8,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -43,11 +44,14 @@ inline double dot3(const V3& a, const V3& b) { return (a.x * b.x + a.y * b.y) + 
 inline double smin_h(double a, double b) { return (b < a) ? b : a; }
 
 constexpr int kSides = 6;      // L, R, B, T, Z (back), F (front)
-// States up to this size are downloaded through pinned memory that the kernel
-// writes (us; six copies to pageable memory behind a kernel / so): 13468 cells
-// 152 / 81, 24000 188 / 105; against 349 and 622 with every field an array of its
-// own and no kernel, 110592 305, 166320 566.
-constexpr size_t kHostRows = (size_t)8 << 20;
+// Host arrays are filled and read through two parts of this size of pinned
+// memory: a kernel gathers or scatters the pairs of one part while the host copies
+// the other.  Measured (us, a copy to or from pageable memory per array and a kernel
+// over all cells / so): state out 1000 cells 117 / 33, 64 k 223 / 172, 216 k 733 / 439,
+// 885 k 3046 / 1728, 3.4 M 15220 / 10965; in 126 / 34, 181 / 105, 442 / 347, 1490 / 1216,
+// 5476 / 4170; gradients out 137 / 33, 581 / 345, 1938 / 975, 9993 / 7436, 37916 / 27786.  Parts
+// of 1/4, 1/2, 1, 2, 4, 8 MiB (885 k cells, state out): 2570, 2031, 1903, 1728, 1791, 2415.
+constexpr size_t kHostPart = (size_t)2 << 20;
 constexpr int kSlots24 = 24;   // AMR-3D face slots per cell (geom/indexing.h:340-372)
 
 }  // namespace
@@ -77,7 +81,9 @@ struct zfv3_ctx {
     double area1[6] = {}, vol1 = 0.0;
     int tab_bcode[6] = {0, 0, 0, 0, 0, 0};
     int tab_per[3] = {0, 0, 0};
-    double* h_rows = nullptr;     // pinned, kHostRows bytes: a small state's rows on their way out
+    double* h_rows = nullptr;     // pinned: rows on their way to or from host arrays (kHostPart)
+    size_t h_bytes = 0;
+    hipEvent_t h_done[2] = {nullptr, nullptr};   // the kernel on each part
     bool use_tables = true;
     int blocks = 0;
     // solver
@@ -98,6 +104,8 @@ struct zfv3_ctx {
         drop_events();
         release();
         if (h_rows) (void)hipHostFree(h_rows);
+        for (hipEvent_t e : h_done)
+            if (e) (void)hipEventDestroy(e);
         if (stream) (void)hipStreamDestroy(stream);
     }
     void drop_events() {
@@ -174,6 +182,65 @@ int read_err(zfv3_ctx* ctx) {
     Z3HIP(hipStreamSynchronize(ctx->stream));
     if (e & 1) return fail(ZFV_ERR_NUMERIC, "numeric error: a flux produced NaN");
     return ZFV_OK;
+}
+
+// The cells of one part of the pinned memory for `rows` rows of host arrays, with
+// that memory there, or 0: an array is device memory, or none can be had.
+int host_part(zfv3_ctx* ctx, const double* const* arrays, int rows) {
+    for (int k = 0; k < rows; ++k) {
+        hipPointerAttribute_t a{};
+        if (arrays[k] && hipPointerGetAttributes(&a, arrays[k]) == hipSuccess && a.type == hipMemoryTypeDevice) return 0;
+    }
+    (void)hipGetLastError();   // pageable memory is unknown to the runtime
+    const size_t row = rows * sizeof(double);
+    const int part = (int)std::min<size_t>(ctx->n, kHostPart / row);
+    const size_t need = (part < ctx->n ? 2 : 1) * part * row;
+    if (part < ctx->n)
+        for (hipEvent_t& e : ctx->h_done)
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                e = nullptr;
+                return 0;
+            }
+    if (ctx->h_bytes < need) {   // the largest so far, at most two parts
+        if (ctx->h_rows) {
+            if (hipStreamSynchronize(ctx->stream) != hipSuccess) return 0;   // a kernel may still read it
+            (void)hipHostFree(ctx->h_rows);
+        }
+        ctx->h_rows = nullptr;
+        ctx->h_bytes = 0;
+        if (hipHostMalloc((void**)&ctx->h_rows, need, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            ctx->h_rows = nullptr;
+            return 0;
+        }
+        ctx->h_bytes = need;
+    }
+    return part;
+}
+
+// Rows m0 to m0 + count - 1 of arrays of pairs into host arrays (null: left out).
+int rows_out(zfv3_ctx* ctx, const double2* q, int m0, int count, int part, double* const* dst) {
+    const int n = ctx->n;
+    auto take = [&](int i) {   // the host's copy of part i
+        const int c0 = i * part, len = std::min(part, n - c0);
+        const double* buf = ctx->h_rows + (size_t)(i & 1) * count * part;
+        for (int k = 0; k < count; ++k)
+            if (dst[k]) std::memcpy(dst[k] + c0, buf + (size_t)k * len, len * sizeof(double));
+    };
+    const int parts = (n + part - 1) / part;
+    for (int i = 0; i < parts; ++i) {
+        const int c0 = i * part, len = std::min(part, n - c0);
+        Z3HIP(launch3_rows(q, n, c0, len, m0, count, ctx->h_rows + (size_t)(i & 1) * count * part, ctx->stream));
+        if (i + 1 < parts) Z3HIP(hipEventRecord(ctx->h_done[i & 1], ctx->stream));
+        if (i > 0) {
+            Z3HIP(hipEventSynchronize(ctx->h_done[(i - 1) & 1]));
+            take(i - 1);
+        }
+    }
+    const int r = read_err(ctx);   // waits for the last part
+    if (r == ZFV_OK || r == ZFV_ERR_NUMERIC) take(parts - 1);
+    return r;
 }
 
 int slot_code(int b) {
@@ -524,12 +591,24 @@ int zfv3_state_upload(zfv3_ctx* ctx, const double* rho, const double* u, const d
     }
     const double* src[6] = {rho, u, v, w, p, e};
     Z3HIP(hipStreamSynchronize(ctx->stream));
-    // on the kernel's stream: from device memory a copy on another one returns
-    // before it is done, and the kernel would not wait for it
-    for (int k = 0; k < 6; ++k)
-        Z3HIP(hipMemcpyAsync(ctx->staging() + k * N, src[k], N * sizeof(double), hipMemcpyDefault, ctx->stream));
-    Z3HIP(launch3_pack(ctx->staging(), ctx->state(ctx->zi), ctx->stream));
-    Z3HIP(hipStreamSynchronize(ctx->stream));   // the arrays are the caller's again
+    const Dev3State z = ctx->state(ctx->zi);
+    if (const int part = host_part(ctx, src, 6)) {
+        for (int c0 = 0, i = 0; c0 < ctx->n; c0 += part, ++i) {
+            const int len = std::min(part, ctx->n - c0);
+            double* buf = ctx->h_rows + (size_t)(i & 1) * 6 * part;
+            if (i >= 2) Z3HIP(hipEventSynchronize(ctx->h_done[i & 1]));   // the part's last kernel has read it
+            for (int k = 0; k < 6; ++k) std::memcpy(buf + (size_t)k * len, src[k] + c0, len * sizeof(double));
+            Z3HIP(launch3_pack(buf, z, c0, len, ctx->stream));
+            if (part < ctx->n) Z3HIP(hipEventRecord(ctx->h_done[i & 1], ctx->stream));
+        }
+    } else {
+        // on the kernel's stream: from device memory a copy on another one returns
+        // before it is done, and the kernel would not wait for it
+        for (int k = 0; k < 6; ++k)
+            Z3HIP(hipMemcpyAsync(ctx->staging() + k * N, src[k], N * sizeof(double), hipMemcpyDefault, ctx->stream));
+        Z3HIP(launch3_pack(ctx->staging(), z, 0, ctx->n, ctx->stream));
+        Z3HIP(hipStreamSynchronize(ctx->stream));   // the arrays are the caller's again
+    }
     ctx->have_state = true;
     return state_changed(ctx);
 }
@@ -539,22 +618,8 @@ int zfv3_state_download(zfv3_ctx* ctx, double* rho, double* u, double* v, double
     if (r) return r;
     const size_t N = (size_t)ctx->n;
     double* dst[6] = {rho, u, v, w, p, e};
-    bool host = 6 * N * sizeof(double) <= kHostRows;
-    for (int k = 0; k < 6 && host; ++k) {
-        hipPointerAttribute_t a{};
-        if (dst[k] && hipPointerGetAttributes(&a, dst[k]) == hipSuccess && a.type == hipMemoryTypeDevice) host = false;
-    }
-    (void)hipGetLastError();   // pageable memory is unknown to the runtime
-    if (host) {
-        if (!ctx->h_rows) Z3HIP(hipHostMalloc((void**)&ctx->h_rows, kHostRows, hipHostMallocDefault));
-        Z3HIP(launch3_rows(ctx->d_z[ctx->zi], ctx->n, 0, 6, ctx->h_rows, ctx->stream));
-        r = read_err(ctx);
-        if (r != ZFV_OK && r != ZFV_ERR_NUMERIC) return r;
-        for (int k = 0; k < 6; ++k)
-            if (dst[k]) std::memcpy(dst[k], ctx->h_rows + k * N, N * sizeof(double));
-        return r;
-    }
-    Z3HIP(launch3_rows(ctx->d_z[ctx->zi], ctx->n, 0, 6, ctx->staging(), ctx->stream));
+    if (const int part = host_part(ctx, dst, 6)) return rows_out(ctx, ctx->d_z[ctx->zi], 0, 6, part, dst);
+    Z3HIP(launch3_rows(ctx->d_z[ctx->zi], ctx->n, 0, ctx->n, 0, 6, ctx->staging(), ctx->stream));
     for (int k = 0; k < 6; ++k)
         if (dst[k])
             Z3HIP(hipMemcpyAsync(dst[k], ctx->staging() + k * N, N * sizeof(double), hipMemcpyDeviceToHost,
@@ -585,9 +650,12 @@ int zfv3_grad_download(zfv3_ctx* ctx, double* g) {
     if (r) return r;
     if (!g) return fail(ZFV_ERR_ARG, "null gradient array");
     const size_t row = 5 * (size_t)ctx->n;
+    double* dst[15];
+    for (int k = 0; k < 15; ++k) dst[k] = g + (size_t)k * ctx->n;
+    if (const int part = host_part(ctx, dst, 15)) return rows_out(ctx, ctx->d_rec, 6, 15, part, dst);
     double* buf = ctx->staging();
     for (int a = 0; a < 3; ++a) {
-        Z3HIP(launch3_rows(ctx->d_rec, ctx->n, 6 + 5 * a, 5, buf, ctx->stream));
+        Z3HIP(launch3_rows(ctx->d_rec, ctx->n, 0, ctx->n, 6 + 5 * a, 5, buf, ctx->stream));
         Z3HIP(hipMemcpyAsync(g + a * row, buf, row * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     }
     return read_err(ctx);

@@ -698,23 +698,24 @@ __global__ void __launch_bounds__(256, (kCorrWaves<FLUX, TAB>)) k3_corr(
     block_min(ctl.next, cand);
 }
 
-// Double m0 + k of every cell, k < count, out of arrays of pairs as rows [k][n].
-__global__ void __launch_bounds__(256) k3_rows(const double2* __restrict__ q, int n, int m0, int count,
-                                               double* __restrict__ out) {
-    const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (c >= n) return;
+// Double m0 + k, k < count, of the cells c0 to c0 + len - 1 out of arrays of pairs,
+// as rows [k][len].
+__global__ void __launch_bounds__(256) k3_rows(const double2* __restrict__ q, int n, int c0, int len, int m0,
+                                               int count, double* __restrict__ out) {
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= len) return;
     const double* v = (const double*)q;
     for (int k = 0; k < count; ++k) {
         const int m = m0 + k;
-        out[(size_t)k * n + c] = v[2 * ((size_t)(m >> 1) * n + c) + (m & 1)];
+        out[(size_t)k * len + i] = v[2 * ((size_t)(m >> 1) * n + c0 + i) + (m & 1)];
     }
 }
 
-// Rows rho, u, v, w, p, e into a state.
-__global__ void __launch_bounds__(256) k3_pack(const double* __restrict__ in, Dev3State z) {
-    const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    const size_t n = (size_t)z.n;
-    if (c < z.n) store3(z, c, Z3{in[c], in[n + c], in[2 * n + c], in[3 * n + c], in[4 * n + c], in[5 * n + c]});
+// Rows [6][len] of rho, u, v, w, p, e into the cells c0 to c0 + len - 1 of a state.
+__global__ void __launch_bounds__(256) k3_pack(const double* __restrict__ in, Dev3State z, int c0, int len) {
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const size_t n = (size_t)len;
+    if (i < len) store3(z, c0 + i, Z3{in[i], in[n + i], in[2 * n + i], in[3 * n + i], in[4 * n + i], in[5 * n + i]});
 }
 
 // Per-workgroup partial sums of V q: mass, momentum x, y, z, energy.
@@ -813,13 +814,13 @@ hipError_t launch3_corr(int flux, const Dev3Mesh& M, const Dev3State& init, cons
     return hipGetLastError();
 }
 
-hipError_t launch3_rows(const double2* q, int n, int m0, int count, double* out, hipStream_t s) {
-    hipLaunchKernelGGL(k3_rows, g256(n), dim3(256), 0, s, q, n, m0, count, out);
+hipError_t launch3_rows(const double2* q, int n, int c0, int len, int m0, int count, double* out, hipStream_t s) {
+    hipLaunchKernelGGL(k3_rows, g256(len), dim3(256), 0, s, q, n, c0, len, m0, count, out);
     return hipGetLastError();
 }
 
-hipError_t launch3_pack(const double* in, const Dev3State& z, hipStream_t s) {
-    hipLaunchKernelGGL(k3_pack, g256(z.n), dim3(256), 0, s, in, z);
+hipError_t launch3_pack(const double* in, const Dev3State& z, int c0, int len, hipStream_t s) {
+    hipLaunchKernelGGL(k3_pack, g256(len), dim3(256), 0, s, in, z, c0, len);
     return hipGetLastError();
 }
 

@@ -82,8 +82,8 @@ hipError_t launch3_grad_pred(int limiter, const Dev3Mesh& M, const Dev3State& in
                              const Eos& eos, const Dev3Ctl& ctl, hipStream_t s);
 hipError_t launch3_corr(int flux, const Dev3Mesh& M, const Dev3State& init, const double2* R, int* wait_out,
                         const Dev3State& next, const Eos& eos, const Dev3Ctl& ctl, hipStream_t s);
-hipError_t launch3_rows(const double2* q, int n, int m0, int count, double* out, hipStream_t s);
-hipError_t launch3_pack(const double* in, const Dev3State& z, hipStream_t s);
+hipError_t launch3_rows(const double2* q, int n, int c0, int len, int m0, int count, double* out, hipStream_t s);
+hipError_t launch3_pack(const double* in, const Dev3State& z, int c0, int len, hipStream_t s);
 hipError_t launch3_totals(const Dev3Mesh& M, const Dev3State& z, double* partial, int nblocks, hipStream_t s);
 
 }  // namespace zfv
