@@ -52,7 +52,7 @@ def kernel_bytes_per_cell(phi):
 # volume and incircle; plus the halo of its tile shape (rows x 62 cells, a
 # two-cell ring of rho, u, v, p and a one-cell ring of e and the counter),
 # which neighbouring tiles read again.
-TILE_ROWS = {512: 6, 768: 10, 1024: 14}
+TILE_ROWS = {256: 2, 512: 6, 768: 10, 1024: 14}
 
 
 def tile_fused_bytes_per_cell(threads):
@@ -121,16 +121,19 @@ WORKLOADS = {
 
 
 # The sources a step kernel is compiled from: its own file and the headers
-# that file includes.
+# that file includes; "tile" and "flux1" are each timed over kernels of two files
+# (the tiled HLL and Rusanov steps, the tiled first-order step).
 STEP_HEADERS = ("zfv_internal.hpp", "zfv_physics.hpp", "zfv_mm.hpp", "zfv_step_common.hpp", "zfv_step_faces.hpp")
 KERNEL_FILES = {"tile": "zfv_tile.hip", "grad_pred": "zfv_kernels.hip", "corr": "zfv_kernels.hip",
                 "flux1": "zfv_kernels.hip", "k3_grad_pred": "zfv_3d.hip", "k3_corr": "zfv_3d.hip",
                 "k3_flux1": "zfv_3d.hip"}
-KERNEL_HEADERS = {"tile": ("zfv_tile.hpp", "zfv_pair.hpp"), "k3_grad_pred": ("zfv_3d.hpp",), "k3_corr": ("zfv_3d.hpp",), "k3_flux1": ("zfv_3d.hpp",)}
+KERNEL_HEADERS = {"tile": ("zfv_tile_flux.hip", "zfv_tile.hpp", "zfv_pair.hpp"),
+                  "flux1": ("zfv_tile.hip", "zfv_tile.hpp", "zfv_pair.hpp"), "k3_grad_pred": ("zfv_3d.hpp",),
+                  "k3_corr": ("zfv_3d.hpp",), "k3_flux1": ("zfv_3d.hpp",)}
 
 
 def kernel_sources_sha(kernel):
-    """Short SHA-256 over the HIP sources a step kernel is compiled from
+    """Short SHA-256 over the sources a step kernel is compiled from
     (which the HBM counter summaries record, so a summary is used only for
     the kernel code it measured); None for a kernel outside the table."""
     import hashlib
@@ -997,7 +1000,7 @@ def main():
     src_sha = kernel_sources_sha(dom)
     # the entry of the launch form in use: kernel, layout, workgroup size
     # (or tile shape), whose register use and access pattern set the bytes
-    lay, blk = ctx.launch(2 if dom == "corr" else 1)
+    lay, blk = ctx.launch({"corr": 2, "flux1": 0}.get(dom, 1))
     tkey = f"{dom}:{lay}:{blk}"
     if os.path.exists(tpath):
         t = json.load(open(tpath)).get(args.workload, {}).get(tkey)
