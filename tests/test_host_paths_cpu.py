@@ -183,6 +183,7 @@ def runs(ctx):
 
 for acc in (1, 2):
     for nx, ny, tiled in ((10000, 1, False), (100000, 1, False), (50000, 4, False), (20000, 10, False), (5000, 4, False),
+                          (1, 1, True), (2, 62, True), (3, 63, True), (7, 125, True), (33, 64, True), (19, 70, True),
                           (8, 8, True), (1, 1000, True), (64, 48, True), (4, 5000, True), (300, 200, True),
                           (900, 700, True)):
         ctx = Z.Context()

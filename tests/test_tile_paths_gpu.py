@@ -55,10 +55,16 @@ def test_tiled_equals_cell_kernels(zfv, acc, flux, bounds, nx, ny):
 
 
 @pytest.mark.parametrize("acc", [1, 2])
-@pytest.mark.parametrize("nx,ny", [(40, 40), (200, 200), (330, 280), (520, 390), (700, 900)])
+@pytest.mark.parametrize("nx,ny", [(40, 40), (200, 200), (330, 280), (450, 420), (520, 390), (700, 900)])
 def test_every_default_shape(zfv, acc, nx, ny):
     ref, til = pair(zfv, nx, ny, (2, 1, 3, 3), acc, "hllc")
     steps_equal(ref, til, 2, f"{acc} {nx}x{ny}")
+
+
+def test_default_shapes_are_all_four(zfv):
+    shapes = {nx: pair(zfv, nx, ny, (2, 1, 3, 3), 2, "hllc")[1].launch(1)
+              for nx, ny in ((40, 40), (200, 200), (330, 280), (450, 420))}
+    assert shapes == {40: (zfv.TILE, 256), 200: (zfv.TILE, 512), 330: (zfv.TILE, 768), 450: (zfv.TILE, 1024)}
 
 
 @pytest.mark.parametrize("acc", [1, 2])
