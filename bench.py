@@ -744,24 +744,25 @@ def ensemble_cpu_baseline(w, sizes, seed, budget_s):
 # array the kernel touches, once (neighbour values served from cache).
 # Slot-major mesh: per slot type + adj (8), face centre (24), area (8) and,
 # for the gradient, the weight (8); cell centre 24, volume 8, incircle 8;
-# state rho, u, v, w, p, e (48); gradients 3 x 5 doubles (120); wait 4.
+# state rho, u, v, w, p, e (48); wait 4; the predictor's record (half state 48,
+# gradients 3 x 5 doubles, counter 8: 176).
 # The first-order update and the corrector also reduce the next step's CFL
 # candidate (incircle, 8), so the standalone reduction runs only after a new
 # state is set.
 CUBE_BYTES_SLOTS = {
     "dt": 40 + 8,
     "flux1": 48 + 6 * 16 + 8 + 48 + 8,
-    "grad_pred": 48 + 24 + 6 * 48 + 4 + 8 + 120 + 48,
-    "corr": 48 + 48 + 120 + 4 + 4 + 24 + 8 + 6 * 40 + 48 + 8,
+    "grad_pred": 48 + 24 + 6 * 48 + 4 + 8 + 176,
+    "corr": 48 + 176 + 4 + 24 + 8 + 6 * 40 + 48 + 8,
 }
 # With the Cuboid's geometry tables (the library's default on a Cuboid) the
-# mesh costs only the incircle per cell: the tables (25 (nx + ny + nz)
+# mesh costs only the incircle per cell: the tables (12 (nx + ny + nz)
 # doubles) stay in cache.
 CUBE_BYTES = {
     "dt": 40 + 8,
     "flux1": 48 + 48 + 8,
-    "grad_pred": 48 + 4 + 120 + 48,
-    "corr": 48 + 48 + 120 + 4 + 4 + 48 + 8,
+    "grad_pred": 48 + 4 + 176,
+    "corr": 48 + 176 + 4 + 48 + 8,
 }
 
 
@@ -937,8 +938,9 @@ def main():
     ctx.synchronize()
 
     if args.copy_calibration:
-        # 5 device-to-device copies of n doubles (the init layer) into fresh
-        # buffers: 8n bytes read and 8n bytes written per copy dispatch.
+        # 3 device-to-device copies of the state (5 arrays of n doubles) into
+        # fresh buffers: 40n bytes read and 40n written per dispatch
+        # (k_state_copy).
         import ctypes as C
         hip = C.CDLL("libamdhip64.so")
         bufs = [C.c_void_p() for _ in range(5)]
@@ -950,7 +952,7 @@ def main():
         ctx.synchronize()
         for b in bufs:
             hip.hipFree(b)
-        print(f"copy calibration: n = {ctx.n} doubles per copy", file=sys.stderr, flush=True)
+        print(f"copy calibration: n = {ctx.n}, 5 n doubles per copy", file=sys.stderr, flush=True)
 
     # timed region: exactly --steps steps, no per-kernel events (an event pair
     # around every launch adds an idle gap between dependent kernels)

@@ -502,8 +502,8 @@ __global__ void __launch_bounds__(256) k3_flux1(Dev3Mesh M, Dev3State in, Dev3St
 // gradient::limiting, gradient.h:412-474) fused with fluxes_stage1
 // (sm_fluid.cpp:176-253) into the records.  The system is diagonal, so the axes are taken one after the
 // other, each with only its own two neighbours in registers and its derivatives
-// stored at once: 129 registers for 190, 96^3 cells with MC 91 -> 69 us, of which
-// the vector instructions take 55.
+// stored at once: 129 registers for 190, 96^3 cells with MC 91 -> 69 us; at 128^3 its
+// vector instructions occupy the SIMDs for 60 % of the time.
 template <int LIM, bool TAB>
 __global__ void __launch_bounds__(256) k3_grad_pred(Dev3Mesh M, Dev3State in, double2* __restrict__ R,
                                                     const int* __restrict__ wait, Eos eos, Dev3Ctl ctl) {
@@ -596,12 +596,13 @@ __global__ void __launch_bounds__(256) k3_grad_pred(Dev3Mesh M, Dev3State in, do
 // the record, written to the array of the next step; returns the next step's
 // CFL candidate of the new state.  The workgroup's cells leave their records in
 // LDS for the neighbours among them (all but a few along z, and along y while
-// nz < 256): with every neighbour read from memory the L1 cache was busy 89 % of
-// the time.  96^3 cells, HLLC: 165 us with one array a field and no LDS, 137 with
-// pairs, 119 so at three waves a SIMD (133 at two; a wave waits for loads 43 % of its
-// time); the vector instructions alone take 87.  Evaluating each face once for
-// both of its cells (tiles marched along x) took 170: with 3D's larger state the
-// exchange costs what it saves.
+// nz < 256): with every neighbour read from memory, a double a load, the L1 cache
+// was busy 85 % of the time at 128^3 (now 73 %).  96^3 cells, HLLC: 165 us with one array a field and no LDS, 137 with
+// pairs, 119 to 123 so at three waves a SIMD (138 at two); at 128^3 its vector
+// instructions occupy the SIMDs for 55 % of the time, and a wave waits for memory 46 %
+// of its.  Evaluating each face once for both of its cells (tiles marched along x)
+// took 180 to 190 where the pairs took 173: with 3D's larger state the exchange
+// costs what it saves.
 template <int FLUX, bool TAB>
 __device__ __forceinline__ double corr_cell(const Dev3Mesh& M, const Dev3State& init, const double2* __restrict__ R,
                                             int* __restrict__ wait_out, const Dev3State& next, const Eos& eos,
