@@ -1,6 +1,7 @@
-"""Spilled registers of the 3D corrector as it was compiled: a bound on the waves
-a SIMD that suits one flux can make another spill by the hundred (HLL 133 ->
-250 us at 96^3 cells) and still give the right results."""
+"""Registers and scratch memory of kernels as they were compiled.  A bound on the
+waves a SIMD that suits one flux can make another spill by the hundred (3D
+corrector, HLL 133 -> 250 us at 96^3 cells) and still give the right results; so
+can an array that the compiler indexes at run time."""
 import os
 import re
 import struct
@@ -28,21 +29,33 @@ def code_objects(path):
         at = data.find(BUNDLE, p)
 
 
-@pytest.mark.skipif(not os.path.exists(READELF), reason="needs llvm-readelf")
-def test_3d_corrector_spills_few_registers(zfv, tmp_path):
-    spills = {}
-    for i, obj in enumerate(code_objects(zfv.LIB_PATH)):
+def metadata(path, tmp_path, part, field):
+    """{kernel: value} of a metadata field of the kernels whose names hold `part`."""
+    out = {}
+    for i, obj in enumerate(code_objects(path)):
+        if part.encode() not in obj:
+            continue
         f = tmp_path / f"{i}.o"
         f.write_bytes(obj)
-        if b"k3_corr" not in obj:
-            continue
         notes = subprocess.run([READELF, "--notes", str(f)], capture_output=True, text=True, check=True).stdout
-        name = None
-        for line in notes.splitlines():
-            m = re.match(r"\s+\.name:\s+(\S*k3_corr\S*)", line)
-            name = m.group(1) if m else (None if re.match(r"\s+\.name:\s+_Z", line) else name)
-            m = re.match(r"\s+\.vgpr_spill_count:\s+(\d+)", line)
-            if m and name:
-                spills[name] = int(m.group(1))
+        for kernel in re.split(r"\n\s+- \.agpr_count", notes)[1:]:
+            name = re.search(r"\.name:\s+(_Z\S+)", kernel).group(1)
+            if part in name:
+                out[name] = int(re.search(rf"\.{field}:\s+(\d+)", kernel).group(1))
+    return out
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="needs llvm-readelf")
+def test_3d_corrector_spills_few_registers(zfv, tmp_path):
+    spills = metadata(zfv.LIB_PATH, tmp_path, "k3_corr", "vgpr_spill_count")
     assert len(spills) == 16, spills   # eight fluxes, tables and slot arrays
     assert max(spills.values()) <= 16, spills
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="needs llvm-readelf")
+def test_mixtures_of_any_size_stay_out_of_scratch(zfv, tmp_path):
+    """The multi-material kernels choose a material by selects, not through a copy
+    of the mixture in scratch memory."""
+    scratch = metadata(zfv.LIB_PATH, tmp_path, "k_mm_", "private_segment_fixed_size")
+    assert sum("k_mm_crpI" in k for k in scratch) == 8, scratch   # one to four materials, both orders
+    assert not any(scratch.values()), {k: v for k, v in scratch.items() if v}

@@ -95,13 +95,23 @@ __device__ __forceinline__ void frac_cutoff(double* b, double eps) {
 constexpr double kFracMinimal = 0x1.0p-54;   // Fractions::minimal = DBL_EPSILON / 4 (fractions.h:14)
 
 // Material idx of a pure cell, by selects (no dynamic indexing of the
-// kernel-argument mixture or of register arrays).
+// kernel-argument mixture or of register arrays).  Value by value: a copied
+// struct becomes a selected address with three and more materials, for which
+// the mixture goes through scratch (208 bytes a lane).
 template <int NM>
 __device__ __forceinline__ Mat pick(const Mix& mx, int idx) {
     Mat r = mx.m[0];
 #pragma unroll
-    for (int i = 1; i < NM; ++i)
-        if (i == idx) r = mx.m[i];
+    for (int i = 1; i < NM; ++i) {
+        const Mat& m = mx.m[i];
+        const bool take = i == idx;
+        r.g = take ? m.g : r.g;
+        r.P0 = take ? m.P0 : r.P0;
+        r.e0 = take ? m.e0 : r.e0;
+        r.Cv = take ? m.Cv : r.Cv;
+        r.T0 = take ? m.T0 : r.T0;
+        r.rho_ref = take ? m.rho_ref : r.rho_ref;
+    }
     return r;
 }
 template <int NM>
