@@ -127,6 +127,11 @@ for call in (up, down):
     less[{row}] = device(8 * n - {short})
     code, kernel = go(call, less)
     assert code == Z.ZFV_ERR_HIP and not kernel
+    one = device(8 * 5 * n)   # the rows of one allocation, and of one that ends in the last row
+    assert go(call, [one + 8 * n * k for k in range(5)]) == (0, True)
+    one = device(8 * 5 * n - {short})
+    code, kernel = go(call, [one + 8 * n * k for k in range(5)])
+    assert code == Z.ZFV_ERR_HIP and not kernel
 """)
 
 

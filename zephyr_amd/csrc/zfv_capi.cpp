@@ -1609,18 +1609,23 @@ static int materialize_grads(zfv_ctx* ctx);
 // doubles, where one kernel can copy them.  Other memory goes through hipMemcpy,
 // which refuses a row that ends before its n-th double.
 static bool on_device(const zfv_ctx* ctx, const double* const* rows, int n) {
+    uintptr_t base = 0;
+    size_t size = 0;   // the allocation of the row before: asked for once where it holds several
     for (int k = 0; k < 5; ++k) {
-        hipPointerAttribute_t a;
-        hipDeviceptr_t base = nullptr;
-        size_t size = 0;
-        if (hipPointerGetAttributes(&a, rows[k]) != hipSuccess || a.type != hipMemoryTypeDevice ||
-            a.device != ctx->device ||
-            hipMemGetAddressRange(&base, &size, const_cast<double*>(rows[k])) != hipSuccess) {
-            (void)hipGetLastError();   // not a HIP allocation
-            return false;
+        const uintptr_t p = (uintptr_t)rows[k];
+        if (p < base || p - base >= size) {
+            hipPointerAttribute_t a;
+            hipDeviceptr_t b = nullptr;
+            if (hipPointerGetAttributes(&a, rows[k]) != hipSuccess || a.type != hipMemoryTypeDevice ||
+                a.device != ctx->device ||
+                hipMemGetAddressRange(&b, &size, const_cast<double*>(rows[k])) != hipSuccess) {
+                (void)hipGetLastError();   // not a HIP allocation
+                return false;
+            }
+            base = (uintptr_t)b;
         }
-        const uintptr_t p = (uintptr_t)rows[k], b = (uintptr_t)base;
-        if (p % sizeof(double) || p < b || p - b > size || (size - (p - b)) / sizeof(double) < (size_t)n) return false;
+        if (p % sizeof(double) || p < base || p - base > size || (size - (p - base)) / sizeof(double) < (size_t)n)
+            return false;
     }
     return true;
 }
